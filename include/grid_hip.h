@@ -140,6 +140,51 @@ int hgrid_fft_pass(const hgrid_pass *p);
 /* Axis lengths the pass kernels support (power of two, 1..1024). */
 int hgrid_fft_supported(long n);
 
+/* ---- tile passes ------------------------------------------------------------------------ */
+
+/* Two kinds of sweep that together cover all axes of a grid (hip/tile_pass.hpp).  The middle axis
+ * is split, n1 = nh * rows (index h rows + l).  A grid in tile form is transformed along x and h
+ * (unnormalised forward), frequencies in natural order:
+ *   A-pass  tile form -> tile form: forward along l and z, kinetic factor, inverse
+ *   B-pass  tile form -> real space, potential factor -> tile form, or one half of that
+ * A 2-D grid has no x: its h takes x's place (flat). */
+typedef struct hgrid_tile {
+  void *psi;             /* device array (complex, precision prec), transformed in place */
+  int prec;              /* HGRID_C128 / HGRID_C64 */
+  long n0, n1, n2;       /* squeezed shape; n2 is contiguous */
+  /* filled in by hgrid_tile_plan */
+  int flat;              /* 2-D: h in x's place */
+  int rows, nh;          /* n1 = nh * rows */
+  long sx, sh;           /* elements between neighbours along x and h */
+  long blocks_a, blocks_b;  /* workgroups of an A-pass and a B-pass (partials per channel) */
+  double back;           /* points along x and h: an inverse after a forward B-pass multiplies by it */
+  /* per pass */
+  unsigned flags;        /* A: PRESCALE, MID_KRED, KIN_REAL, KCUT, POST_RED
+                          * B: PRESCALE, PRE_VEFF, PRE_RED, POT_NOFFT1, POT_NOFFT2, POST_RED */
+  const void *twx, *twl, *twz, *twy;  /* exp(-2 pi i m / n) of x (2-D: h), rows, n2 and n1 */
+  const double *scale;
+  double post;           /* A: real factor applied to the input */
+  const void *ktab_0, *ktab_1, *ktab_2;   /* kinetic tables (double2) per axis, natural order */
+  const double *k2_0, *k2_1;              /* |k|^2 for MID_KRED; z's is formed from k2_dk */
+  double k2_dk;
+  const double *kc_0, *kc_1, *kc_2;       /* (k - k0)^2 for KCUT */
+  double kcut2;
+  const void *pot;       /* complex potential (NULL: none) */
+  const double *vext;
+  double *veff;          /* V_eff in the order of the B-pass's threads (n0 n1 n2 doubles) */
+  double g, c_re, c_im, cons;
+  double *partials;
+} hgrid_tile;
+
+enum { HGRID_TILE_KINETIC = 0,   /* A-pass */
+       HGRID_TILE_START = 1,     /* B-pass: inverse, V_eff / reductions, nothing else stored */
+       HGRID_TILE_POT = 2,       /* B-pass with a complex potential or none */
+       HGRID_TILE_GPE = 3 };     /* B-pass with V_eff, or vext where veff is NULL; c real or imaginary */
+
+/* Whether tile passes cover this shape and precision; fills in the geometry. */
+int hgrid_tile_plan(int prec, long n0, long n1, long n2, hgrid_tile *t);
+int hgrid_tile_pass(const hgrid_tile *t, int pass);
+
 /* ---- reductions ------------------------------------------------------------------------- */
 
 /* out[c] = sum_{b < nblocks} partials[c * nblocks + b] for c < nchan, deterministic order,

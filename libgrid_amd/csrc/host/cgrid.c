@@ -164,18 +164,25 @@ static void download(cgrid *g) {
   d->valid |= GV_HOST;
 }
 
-/* Transform a state left along the contiguous axis by a fused step back to real space
- * (unnormalised inverse: the step's kinetic factor already carried 1/N). */
+/* Transform a state left transformed by a fused step back to real space (unnormalised inverse:
+ * the step's kinetic factor already carried 1/N). */
 void lg_c_materialize(cgrid *g) {
   grid_dev *d = g->dev;
   if (d->kpend) lg_fatal("internal: a merged relaxation batch left its state between kinetic half-steps");
   if (!d->zpend) return;
   lg_shape s;
   lg_squeeze(g->nx, g->ny, g->nz, &s);
-  hgrid_pass p;
-  lg_pass_init(&p, &s, d->prec, d->d, d->d, 2);
-  p.dir1 = +1;
-  lg_run_pass(&p);
+  if (d->zpend == 2) {
+    hgrid_tile t;
+    if (!lg_tile_init(&t, &s, d->prec, d->d)) lg_fatal("internal: a grid in tile form that tile passes do not cover");
+    t.flags = HGRID_PF_POT_NOFFT2;
+    lg_run_tile(&t, HGRID_TILE_POT);
+  } else {
+    hgrid_pass p;
+    lg_pass_init(&p, &s, d->prec, d->d, d->d, 2);
+    p.dir1 = +1;
+    lg_run_pass(&p);
+  }
   d->zpend = 0;
 }
 
@@ -286,6 +293,7 @@ void cgrid_set_precision(cgrid *grid, char prec) {
   grid_dev *d = grid->dev;
   if (d->prec == p) return;
   d->stamp++;
+  if (d->zpend == 2) lg_c_materialize(grid); /* the other precision's tile passes need not cover the shape */
   if (lg_prec_size(p) == lg_prec_size(d->prec)) {
     /* FP32 storage either way: only the arithmetic of the passes changes */
     d->prec = p;

@@ -88,20 +88,54 @@ INT grid_hip_pass_times(INT max, int *axis, int *nfft, unsigned *flags, long *le
   return n;
 }
 
-void lg_run_pass(hgrid_pass *p) {
+static pass_record *trace_begin(void) {
   pass_record *r = (g_trace_on && g_trace_n < LG_PASS_TRACE_MAX) ? &g_trace[g_trace_n++] : NULL;
   if (r) lg_hip(hgrid_event_record(r->ev[0]), "hipEventRecord (pass timing)");
+  return r;
+}
+
+static void trace_end(pass_record *r, int axis, int nfft, unsigned flags, long len, int prec) {
+  if (!r) return;
+  lg_hip(hgrid_event_record(r->ev[1]), "hipEventRecord (pass timing)");
+  r->axis = axis;
+  r->nfft = nfft;
+  r->flags = flags;
+  r->len = len;
+  r->prec = prec;
+}
+
+void lg_run_pass(hgrid_pass *p) {
+  pass_record *r = trace_begin();
   int rc = hgrid_fft_pass(p);
   if (rc) lg_fatal("FFT pass (axis %d, shape %ld x %ld x %ld) failed: %s", p->axis, p->n0, p->n1, p->n2,
                    hgrid_last_error()[0] ? hgrid_last_error() : "unsupported configuration");
-  if (r) {
-    lg_hip(hgrid_event_record(r->ev[1]), "hipEventRecord (pass timing)");
-    r->axis = p->axis;
-    r->nfft = p->nfft;
-    r->flags = p->flags;
-    r->len = p->axis == 0 ? p->n0 : p->axis == 1 ? p->n1 : p->n2;
-    r->prec = p->prec;
-  }
+  trace_end(r, p->axis, p->nfft, p->flags, p->axis == 0 ? p->n0 : p->axis == 1 ? p->n1 : p->n2, p->prec);
+}
+
+/* ---- tile passes ---------------------------------------------------------------------------- */
+
+int lg_tile_init(hgrid_tile *t, const lg_shape *s, int prec, void *psi) {
+  if (s->m < 2 || !hgrid_tile_plan(prec, s->n[0], s->n[1], s->n[2], t)) return 0;
+  t->psi = psi;
+  t->twx = lg_twiddles(t->flat ? t->nh : t->n0, prec);
+  t->twl = lg_twiddles(t->rows, prec);
+  t->twz = lg_twiddles(t->n2, prec);
+  t->twy = lg_twiddles(t->n1, prec);
+  return 1;
+}
+
+/* recorded by the pass timing as axis 3 (A-pass) and 4 (B-pass) */
+void lg_run_tile(hgrid_tile *t, int pass) {
+  pass_record *r = trace_begin();
+  if (hgrid_tile_pass(t, pass))
+    lg_fatal("tile pass %d (shape %ld x %ld x %ld) failed: %s", pass, t->n0, t->n1, t->n2,
+             hgrid_last_error()[0] ? hgrid_last_error() : "unsupported configuration");
+  unsigned flags = t->flags;
+  if (pass == HGRID_TILE_KINETIC) flags |= HGRID_PF_MID_KIN;
+  else if (pass == HGRID_TILE_START) flags |= HGRID_PF_PRE_AFTER | HGRID_PF_NOSTORE;
+  else flags |= pass == HGRID_TILE_GPE ? HGRID_PF_MID_GPE : t->pot ? HGRID_PF_MID_POT : 0;
+  trace_end(r, pass == HGRID_TILE_KINETIC ? 3 : 4, flags & (HGRID_PF_NOSTORE | HGRID_PF_POT_NOFFT1 | HGRID_PF_POT_NOFFT2) ? 1 : 2,
+            flags, pass == HGRID_TILE_KINETIC ? t->rows * t->n2 : (long)t->back, t->prec);
 }
 
 static void copy_scaled(void *in, void *out, int prec, long n, double post, const double *scale) {

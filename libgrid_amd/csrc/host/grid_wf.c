@@ -9,7 +9,8 @@
  * a grid with at least two non-trivial axes it runs as 2 * m + 3 pencil passes (9 for 3-D):
  * the kinetic factor sits between a forward and an inverse transform of the outermost axis,
  * the potential factor between an inverse and a forward transform of the contiguous axis,
- * and the 1/N of both normalised inverse transforms is folded into the kinetic tables.
+ * and the 1/N of both normalised inverse transforms is folded into the kinetic tables.  Grids that
+ * the tile passes cover take 3 passes instead, after a first one (tile_step).
  */
 #include "internal.h"
 #include "relax_rule.h"
@@ -309,7 +310,166 @@ typedef struct {
   int stage;
 } step_args;
 
+static const void *sq(void *const t[3], const lg_shape *s, const cgrid *g, int a) {
+  return t[s->phys[a] >= 0 ? s->phys[a] : trivial_phys(g)];
+}
+
+/* The step in tile passes (hip/tile_pass.hpp), where they cover the grid: A-passes K, a B-pass V,
+ * and the state left in tile form.  Entering from real space costs one more B-pass (forward
+ * transforms along x and h), a result in real space another.  The same step_args, tables and
+ * reductions as the pencil form below. */
+static int tile_step(wf *gwf, const step_args *sa) {
+  cgrid *g = gwf->grid;
+  grid_dev *d = g->dev;
+  lg_shape s;
+  lg_squeeze(g->nx, g->ny, g->nz, &s);
+  hgrid_tile base, t;
+  /* complex time with a real potential stays with the pencils */
+  if ((sa->gpe && sa->c_re != 0.0 && sa->c_im != 0.0) || !lg_tile_init(&base, &s, d->prec, NULL)) return 0;
+  const double *scale;
+  base.psi = lg_c_raw(g, &scale);
+  const int defer = !sa->no_defer, stage = sa->stage;
+  if (stage && (!defer || sa->gpe != 1 || sa->g != 0.0 || (stage >= 2 && (d->zpend != 2 || !d->kpend || sa->want_energy))))
+    lg_fatal("internal: merged relaxation stage %d on a state it does not apply to", stage);
+  if (stage <= 1 && d->kpend) lg_fatal("internal: a merged relaxation batch was left unfinished");
+  if (!defer && (sa->want_post_norm || sa->want_energy)) lg_fatal("internal: reductions of a step that ends in real space");
+  if (d->zpend == 1 || (d->zpend && !defer)) lg_c_materialize(g);
+  const int tin = d->zpend == 2;
+  ktab_cache *kt = stage == 2 ? lg_kinetic_tables_in(g, &d->kin2, 2.0 * sa->tm_re, 2.0 * sa->tm_im, g->fft_norm)
+                              : lg_kinetic_tables(g, sa->tm_re, sa->tm_im, g->fft_norm);
+  ktab_cache *k2 = sa->want_energy ? lg_k2_tables(g) : NULL;
+  const int veff = sa->gpe && sa->g != 0.0;
+  if (veff && !d->rho) lg_hip(hgrid_malloc((void **)&d->rho, d->n * sizeof(double)), "hipMalloc (density)");
+  const long nbA = base.blocks_a, nbB = base.blocks_b, nbP = nbA > nbB ? nbA : nbB;
+  double *partB = lg_partials(HGRID_RED_NCHAN * (nbB + nbA + nbP));
+  double *partK = partB + HGRID_RED_NCHAN * nbB, *partP = partK + HGRID_RED_NCHAN * nbA;
+  const double *pend = scale; /* the pending scale, until a pass that stores has applied it */
+  double post = 1.0;
+
+  /* start of the step: V_eff and the input's reductions */
+  if (stage < 2 && (veff || sa->want_energy)) {
+    t = base;
+    t.flags = tin ? 0 : HGRID_PF_POT_NOFFT1;
+    if (scale) { t.flags |= HGRID_PF_PRESCALE; t.scale = scale; }
+    t.vext = sa->vext;
+    t.g = sa->g;
+    if (veff) { t.flags |= HGRID_PF_PRE_VEFF; t.veff = d->rho; }
+    if (sa->want_energy) { t.flags |= HGRID_PF_PRE_RED; t.partials = partB; }
+    lg_run_tile(&t, HGRID_TILE_START);
+  }
+  if (!tin) {
+    /* into tile form; the 4th-order step's first V(t/6) before it */
+    t = base;
+    t.flags = HGRID_PF_POT_NOFFT1;
+    if (pend) { t.flags |= HGRID_PF_PRESCALE; t.scale = pend; }
+    pend = NULL;
+    t.pot = sa->pot6;
+    t.c_re = sa->c6_re;
+    t.c_im = sa->c6_im;
+    t.cons = sa->cons;
+    lg_run_tile(&t, HGRID_TILE_POT);
+  } else if (stage < 2) {
+    /* the forward B-pass of the real-space state, which the stored form replaces, would have given
+     * `back` times the stored values; the kinetic factors' 1/N accounts for the round trip */
+    post = base.back;
+  }
+  hgrid_finalize fin;
+  memset(&fin, 0, sizeof(fin));
+  if (sa->want_energy) {
+    hgrid_reduce_job j = {partB, nbB, HGRID_RED_NORM, 3, d->dscal + GS_RED};
+    fin.job[fin.njobs++] = j;
+  }
+  long nbpost = nbA;
+  for (int half = 0; half < 2; ++half) {
+    if ((stage == 1 || stage == 2) && half == 1) break;
+    if (stage == 3 && half == 0) continue;
+    t = base;
+    if (pend) { t.flags |= HGRID_PF_PRESCALE; t.scale = pend; }
+    pend = NULL;
+    t.post = post;
+    post = 1.0;
+    if (sa->tm_im == 0.0) t.flags |= HGRID_PF_KIN_REAL;
+    t.ktab_0 = sq(kt->t, &s, g, 0);
+    t.ktab_1 = sq(kt->t, &s, g, 1);
+    t.ktab_2 = sq(kt->t, &s, g, 2);
+    if (sa->kcut) {
+      t.flags |= HGRID_PF_KCUT;
+      t.kc_0 = sq((void *const *)kt->kc, &s, g, 0);
+      t.kc_1 = sq((void *const *)kt->kc, &s, g, 1);
+      t.kc_2 = sq((void *const *)kt->kc, &s, g, 2);
+      t.kcut2 = sa->kcut2;
+    }
+    if (half == 0 && sa->want_energy) {
+      t.flags |= HGRID_PF_MID_KRED;
+      t.k2_0 = sq((void *const *)k2->k2, &s, g, 0);
+      t.k2_1 = sq((void *const *)k2->k2, &s, g, 1);
+      t.k2_dk = 2.0 * M_PI / (g->step * (double)s.n[2]); /* the same expression as lg_k2_tables */
+      t.partials = partK;
+      hgrid_reduce_job j = {partK, nbA, HGRID_RED_KIN, 1, d->dscal + GS_RED + HGRID_RED_KIN};
+      fin.job[fin.njobs++] = j;
+    }
+    if (half == 1 && sa->want_post_norm) {
+      /* sum |S|^2 of the result in tile form: `back` times less than the real-space sum (Parseval);
+       * the finalize multiplies it in */
+      t.flags |= HGRID_PF_POST_RED;
+      t.partials = partP;
+    }
+    lg_run_tile(&t, HGRID_TILE_KINETIC);
+    if (half == 0) {
+      if (sa->gpe || sa->pot) {
+        t = base;
+        t.c_re = sa->c_re;
+        t.c_im = sa->c_im;
+        t.cons = sa->cons;
+        if (sa->gpe) {
+          t.veff = veff ? d->rho : NULL;
+          t.vext = sa->vext;
+        } else {
+          t.pot = sa->pot;
+        }
+        if ((stage == 1 || stage == 2) && sa->want_post_norm) {
+          t.flags |= HGRID_PF_POST_RED;
+          t.partials = partP;
+          nbpost = nbB;
+        }
+        lg_run_tile(&t, sa->gpe ? HGRID_TILE_GPE : HGRID_TILE_POT);
+      } else {
+        post = base.back; /* inverse and forward B-pass with nothing between them */
+      }
+    }
+  }
+  if (!defer) {
+    t = base;
+    t.flags = HGRID_PF_POT_NOFFT2;
+    t.pot = sa->pot6;
+    t.c_re = sa->c6_re;
+    t.c_im = sa->c6_im;
+    t.cons = sa->cons;
+    lg_run_tile(&t, HGRID_TILE_POT);
+  }
+  if (sa->want_post_norm) {
+    hgrid_reduce_job j = {partP, nbpost, HGRID_RED_POST, 1, d->dscal + GS_RED + HGRID_RED_POST};
+    fin.job[fin.njobs++] = j;
+  }
+  if (sa->renorm_target > 0.0) {
+    fin.scale = d->dscal + GS_SCALE;
+    fin.norm_sum = d->dscal + GS_RED + HGRID_RED_POST;
+    fin.target = sa->renorm_target;
+    fin.dv = lg_step_factor(g->nx, g->ny, g->nz, g->step) * base.back;
+  } else if (scale) {
+    fin.scale = d->dscal + GS_SCALE; /* the pending scale was applied */
+  }
+  if (fin.njobs || fin.scale) lg_hip(hgrid_step_finalize(&fin), "step_finalize");
+  d->valid = GV_DEV;
+  d->stamp++;
+  d->pending = sa->renorm_target > 0.0;
+  d->zpend = defer ? 2 : 0;
+  d->kpend = stage == 1 || stage == 2;
+  return 1;
+}
+
 static void fused_step(wf *gwf, const step_args *sa) {
+  if (tile_step(gwf, sa)) return;
   cgrid *g = gwf->grid;
   grid_dev *d = g->dev;
   lg_shape s;
@@ -327,7 +487,7 @@ static void fused_step(wf *gwf, const step_args *sa) {
   if (stage && (!defer || sa->gpe != 1 || sa->g != 0.0 || (stage >= 2 && (!d->zpend || !d->kpend || sa->want_energy))))
     lg_fatal("internal: merged relaxation stage %d on a state it does not apply to", stage);
   if (stage <= 1 && d->kpend) lg_fatal("internal: a merged relaxation batch was left unfinished");
-  if (d->zpend && !defer) lg_c_materialize(g);
+  if (d->zpend == 2 || (d->zpend && !defer)) lg_c_materialize(g);
   const int zin = d->zpend;
   /* stage 2 applies the kinetic factor of a whole step: the tables of twice the half-step time
    * (one unnormalised round trip per step, so one 1/N) */

@@ -37,9 +37,10 @@ typedef struct grid_dev {
   void *d;                 /* device array, or NULL */
   int valid;               /* GV_HOST | GV_DEV */
   int pending;             /* device scale slot differs from 1 */
-  int zpend;               /* the device array holds the unnormalised forward transform of the
-                              state along the squeezed contiguous axis (fused steps leave it so
-                              between steps); accessors transform back before other use */
+  int zpend;               /* the device array holds an unnormalised forward transform of the state
+                              (fused steps leave it so between steps): 1 along the squeezed
+                              contiguous axis, 2 tile form (hip/tile_pass.hpp); accessors transform
+                              back before other use */
   double *dscal;           /* GS_N device doubles */
   /* wavefunction helpers (complex grids used as wf->grid) */
   void *work;              /* device-only scratch of the same size (kinetic energy etc.) */
@@ -79,7 +80,7 @@ void lg_c_written(cgrid *g, int scale_consumed);
 void lg_c_set_pending(cgrid *g, double re, double im); /* multiply the pending scale */
 void lg_c_flush(cgrid *g);
 void *lg_c_raw(cgrid *g, const double **scale);  /* device data as stored (zpend kept), for the fused step */
-void lg_c_materialize(cgrid *g);                 /* undo zpend: inverse transform along the contiguous axis */
+void lg_c_materialize(cgrid *g);                 /* undo zpend: inverse transform to real space */
 void lg_c_host_sync(cgrid *g);
 grid_dev *lg_rdev(rgrid *g);
 const double *lg_r_in(rgrid *g);
@@ -98,6 +99,9 @@ typedef struct lg_shape {
 void lg_squeeze(long nx, long ny, long nz, lg_shape *s);
 void lg_pass_init(hgrid_pass *p, const lg_shape *s, int prec, void *in, void *out, int axis);
 void lg_run_pass(hgrid_pass *p);
+/* tile passes of a squeezed shape: 0 if they do not cover it; fills in geometry and twiddles */
+int lg_tile_init(hgrid_tile *t, const lg_shape *s, int prec, void *psi);
+void lg_run_tile(hgrid_tile *t, int pass);
 /* forward / inverse 3-D transform of one device array through the pass kernels */
 void lg_fft_forward(void *in, void *out, int prec, const lg_shape *s, const double *scale);
 void lg_fft_inverse(void *in, void *out, int prec, const lg_shape *s, double post, const double *scale);

@@ -1,0 +1,105 @@
+"""Tile passes (csrc/hip/tile_pass.hpp): the shapes they take, and steps on every tile geometry
+against the oracle.
+
+Bars of the GPU steps, fixed by the number of roundings: two steps are 8 transforms of at most 2^22
+points, each about log2 N roundings in a row, 8 * 22 * eps / 2 with eps = 1.1e-16 or 6e-8 in the
+worst case of all rounding the same way; 2e-14 and 1e-5.  A wrong index, twiddle or factor is of
+order 1."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import libgrid_amd as LG
+from conftest import rel_l2
+
+LENGTHS = (16, 24, 32, 48, 64, 96, 128, 192, 256)
+BARS = {b"\x00": 2e-14, b"\x01": 1e-5}
+
+
+def planned(prec, n0, n1, n2):
+    lib = LG.load()
+    lib.hgrid_tile_plan.restype = C.c_int
+    lib.hgrid_tile_plan.argtypes = [C.c_int, C.c_long, C.c_long, C.c_long, C.c_void_p]
+    return bool(lib.hgrid_tile_plan(prec, n0, n1, n2, C.create_string_buffer(1024)))
+
+
+def test_shapes_taken_and_left():
+    for n in LENGTHS[2:]:
+        for prec in (LG.HGRID_C128, LG.HGRID_C64):
+            assert planned(prec, n, n, n), (prec, n)
+        assert not planned(LG.HGRID_C64X, n, n, n)  # FP32 storage with FP64 arithmetic
+    assert planned(LG.HGRID_C128, 1, 384, 512) and planned(LG.HGRID_C64, 1, 1024, 64)
+    for shape in ((8, 64, 64), (64, 12, 64), (64, 64, 512), (512, 64, 64), (64, 512, 64), (1, 1, 64), (1, 32, 64),
+                  (64, 384, 64), (1, 64, 24)):
+        assert not planned(LG.HGRID_C128, *shape), shape
+
+
+def steps(lg, orc, shape):
+    """Errors of two steps of each kind: imaginary and real time with a real potential (with and
+    without the density), real time with a complex one (plain, with cutoff, 4th order)."""
+    rng = np.random.default_rng(sum(shape))
+    step, mass = 0.3, 1.2
+    psi = (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) * 0.3 + 1.0
+    psi /= np.sqrt(np.sum(np.abs(psi) ** 2) * step ** sum(n > 1 for n in shape))
+    v = rng.uniform(0, 1, shape)
+    pot = (v + 0.05j * rng.uniform(0, 1, shape)).astype(np.complex128)
+    kmax = 0.6 * np.sqrt(sum((np.pi / step) ** 2 for n in shape if n > 1))
+    k0 = (0.2, -0.1, 0.3)
+
+    def run(prec, prop, one):
+        w = lg.grid_wf_alloc(*shape, step, mass, LG.WF_PERIODIC_BOUNDARY, prop, b"w")
+        w.contents.kmax = kmax
+        LG.set_cgrid(w.contents.grid, psi)
+        lg.cgrid_set_momentum(w.contents.grid, *k0)
+        lg.cgrid_set_precision(w.contents.grid, prec)
+        for _ in range(2):
+            one(w)
+        out = LG.get_cgrid(w.contents.grid)
+        lg.grid_wf_free(w)
+        return out
+
+    vr = lg.rgrid_alloc(*shape, step, LG.boundary("rgrid_value_outside_periodic"), None, b"v")
+    LG.set_rgrid(vr, v)
+    vp = lg.cgrid_alloc(*shape, step, LG.boundary("cgrid_value_outside_periodic"), None, b"pot")
+    LG.set_cgrid(vp, pot)
+    for g, time, norm in ((0.3, -0.05j, 1), (0.0, -0.05j, 1), (0.3, 0.03, 0), (0.3, 0.03 - 0.02j, 0)):
+        ref = psi.copy()
+        for _ in range(2):
+            orc.gpe_step_inplace(ref, v, g, step, mass, k0, time, normalize=bool(norm))
+        for prec, bar in BARS.items():
+            got = run(prec, LG.WF_2ND_ORDER_FFT, lambda w: lg.grid_wf_gpe_propagate(w, vr, g, LG.c_complex.of(time), norm))
+            yield f"gpe g {g} t {time} precision {prec[0]}", rel_l2(got, ref), bar
+    for prop, name in ((LG.WF_2ND_ORDER_FFT, ""), (LG.WF_2ND_ORDER_CFFT, "cfft_"), (LG.WF_4TH_ORDER_FFT, "4th_")):
+        ref = psi.copy()
+        for _ in range(2):
+            getattr(orc, f"wf_propagate_{name}inplace")(ref, pot, step, mass, k0, 0.02, *([kmax] if "cfft" in name else []))
+        for prec, bar in BARS.items():
+            got = run(prec, prop, lambda w: lg.grid_wf_propagate(w, vp, LG.c_complex.of(0.02)))
+            yield f"propagate {name} precision {prec[0]}", rel_l2(got, ref), bar
+    lg.cgrid_free(vp)
+    lg.rgrid_free(vr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n1", LENGTHS)
+@pytest.mark.parametrize("axis", ["x", "z"])
+def test_every_tile_geometry(lg, orc, axis, n1):
+    """Every (x, h) geometry of the B-pass and every (z, rows) geometry of the A-pass."""
+    for n in LENGTHS:
+        shape = (n, n1, 16) if axis == "x" else (16, n1, n)
+        print(f"[case] {shape}", flush=True)
+        for what, err, bar in steps(lg, orc, shape):
+            assert err < bar, f"{shape} {what}: rel L2 {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n1", (64, 96, 128, 192, 256, 384, 512, 768, 1024))
+def test_every_2d_geometry(lg, orc, n1):
+    for n2 in (32, 48, 64, 96, 384, 512):
+        for shape in ((1, n1, n2), (n1, 1, n2)):
+            if n1 == 768 or (n2 == 48 and n1 < 128):  # 768 is no FFT length
+                continue
+            print(f"[case] {shape}", flush=True)
+            for what, err, bar in steps(lg, orc, shape):
+                assert err < bar, f"{shape} {what}: rel L2 {err:.3e}"
