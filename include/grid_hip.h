@@ -322,14 +322,13 @@ int hgrid_b2d_launch(const hgrid_b2d_job *jobs, int njobs, int *queue, int varia
 int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void *w, const float *bias, void *y, int ys, int yo,
                    int cout, const void *mask, int mks, int mko, int lgS, long nvox, int relu);
 /* partial[p][co][t][ci] of dW = sum_m dy[m][dyo + co] x[m + d_t][xo + ci]; sum the
- * hgrid_nn_wgrad_partials(nvox) partials with hgrid_nn_reduce.  bpartial (may be NULL)
- * receives [chunk][co] column sums of dy (the bias gradient), hgrid_nn_wgrad_chunks(nvox)
+ * hgrid_nn_wgrad_partials(nvox, lgS) partials with hgrid_nn_reduce.  bpartial (may be NULL)
+ * receives [chunk][co] column sums of dy (the bias gradient), hgrid_nn_wgrad_chunks(nvox, lgS)
  * rows. */
 int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, const void *x, int xs, int xo, int cin, int lgS,
                          long nvox, float *partial, float *bpartial);
-long hgrid_nn_wgrad_chunks(long nvox);
-long hgrid_nn_wgrad_partials(long nvox);
-long hgrid_nn_wgrad_chunk(long nvox);
+long hgrid_nn_wgrad_chunks(long nvox, int lgS);
+long hgrid_nn_wgrad_partials(long nvox, int lgS);
 int hgrid_nn_reduce(const float *partial, long np, long n, float *out, int accumulate);
 int hgrid_nn_reduce_strided(const float *partial, long np, int stride, int ncols, float *out);
 /* partial[chunk][c] = column sums of d[.][dof + c]; hgrid_nn_colsum_chunks(nvox) chunks */

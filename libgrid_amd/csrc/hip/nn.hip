@@ -218,19 +218,212 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad(const bf16 *__restrict__ dy
       }
 }
 
-// out[e] = sum_p partial[p][e] in order p = 0, 1, ... (deterministic); accumulate adds to out
-__global__ void k_reduce(const float *__restrict__ partial, long np, long n, float *__restrict__ out, int accumulate) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  // eight independent running sums (partials p = 8k + i go to sum i), added in a fixed order
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  long p = 0;
-  for (; p + 8 <= np; p += 8)
+// The same for cubes of side 8 to 64 (64^3, 8 samples: 48 -> 16 and 8 -> 16 channels 1321 -> 229 us on
+// average, the other layers 180 -> 62; the whole minibatch 11.2 -> 6.8 ms), with X read from memory about four times instead of once per
+// tap.  Grid (chunks, Cin / 16, Cout / (16 CT)).  Per step a workgroup stages BV voxels of dY (whole
+// rows of one z) and the rows of X that all 27 taps of them touch, 3 planes x (rows + 2), as
+// [voxel][16 channels], straight copies; both operands need 8 voxels of one channel per lane, which
+// the transposing LDS reads give (ds_read_b64_tr_b16: each 16 lanes read 4 rows of 16 channels
+// and lane c gets channel c of the 4).  A tap is then an address: its row offset, and the x of each
+// lane wrapped.  The next step's global loads are in flight during the products.
+// CT = 1: each of the 4 waves takes a quarter of the voxels and all taps (27 tiles of 16 x 16).
+// CT = 2: waves 0, 2 and 1, 3 take half of the voxels each; waves 0, 1 the first 5 of the 9 (dz, dy)
+// and waves 2, 3 the others, for two tiles of 16 output channels, which share the X operand.
+// The waves' sums are added through LDS in a fixed order: one partial per chunk.
+// Bound by the LDS reads of X (two 512-byte reads per product, 8 cycles of the CU's LDS against 16 of
+// a SIMD's matrix core).
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 *lds4;
+
+__device__ __forceinline__ bf16x8 tr8(const bf16 *lo, const bf16 *hi) {
+  union {
+    s16x4 h[2];
+    bf16x8 v;
+  } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)lo);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)hi);
+  return u.v;
+}
+
+template <int LGS> struct WRows {
+  static constexpr int S = 1 << LGS, RB = S >= 32 ? 256 / S : S, BV = RB * S;  // rows and voxels per step
+  static constexpr int XV = 3 * (RB + 2) * S;                                  // staged voxels of X
+  static_assert(LGS >= 3 && LGS <= 6, "a step is whole rows of one plane");
+};
+
+template <int LGS, int CT>
+__global__ void __launch_bounds__(256, 2) k_wgrad_rows(const bf16 *__restrict__ dy, int dys, int dyo,
+                                                       const bf16 *__restrict__ x, int xs, int xo, int cin, long nvox,
+                                                       long vc, int cout, float *__restrict__ partial,
+                                                       float *__restrict__ bpartial) {
+  using G = WRows<LGS>;
+  constexpr int S = G::S, RB = G::RB, BV = G::BV, XV = G::XV, NK = BV / 32;  // NK: products' K steps of 32 voxels
+  constexpr int KW = CT == 1 ? 4 : 2;                                        // waves that share the voxels
+  constexpr int NC = CT == 1 ? 9 : 5;                                        // (dz, dy) per wave
+  constexpr int XC = XV * 2, YC = BV * 2 * CT;                               // 16-byte pieces per step
+  constexpr int XL = (XC + 255) / 256, YL = (YC + 255) / 256;
+  constexpr int STAGE = XV * 16 + CT * BV * 16;
+  constexpr int SUMS = (CT == 1 ? 28 : 31) * CT * 256 * 2;  // the waves' sums, in bf16 units: taps and bias
+  __shared__ __align__(16) bf16 lds[STAGE > SUMS ? STAGE : SUMS];
+  bf16 *xl = lds, *yl = lds + XV * 16;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, r = lane & 15;
+  const int kw = wave % KW, th = wave / KW;
+  const int ci0 = blockIdx.y * 16, co0 = blockIdx.z * 16 * CT;
+  const int half_ok = cin - ci0 >= 16 ? 2 : 1;  // Cin = 8: the upper half of the tile is zero
+  const long v0 = (long)blockIdx.x * vc, v1 = v0 + vc < nvox ? v0 + vc : nvox;
+  // LDS element of this lane in a K step's transposed read at x shift dx: voxel 8 g + 4 h + r / 4, channels 4 (r % 4)..
+  constexpr int SEG = S == 64 ? 2 : 1;  // K steps per row
+  int off[SEG][2][3];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s[i] += partial[(p + i) * n + e];
-  for (int i = 0; p < np; ++p, ++i) s[i] += partial[p * n + e];
-  const float t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
-  out[e] = accumulate ? out[e] + t : t;
+  for (int sg = 0; sg < SEG; ++sg)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int n = 32 * sg + 8 * g + 4 * h + (r >> 2);
+        off[sg][h][d] = ((n / S) * S + ((n + d - 1) & (S - 1))) * 16 + 4 * (r & 3);
+      }
+  const int yoff = (8 * g + (r >> 2)) * 16 + 4 * (r & 3);
+  bf16x8 px[XL], py[YL];
+  auto fetch = [&](long m0) {
+    // addresses are formed anew each step instead of being kept in registers across the products
+    int t = tid;
+    __asm__ volatile("" : "+v"(t));
+    const long bz = (m0 >> (3 * LGS)) << (3 * LGS);
+    const int z = (int)((m0 >> (2 * LGS)) & (S - 1)), y0 = (int)((m0 >> LGS) & (S - 1));
+#pragma unroll
+    for (int k = 0; k < XL; ++k) {
+      const int e = t + 256 * k, half = e & 1, v = e >> 1;
+      const int p = v / ((RB + 2) * S), row = (v >> LGS) % (RB + 2), xx = v & (S - 1);
+      px[k] = zero8();
+      if ((XC % 256 == 0 || e < XC) && half < half_ok) {
+        const long m = bz + ((long)((z + p - 1) & (S - 1)) << (2 * LGS)) + (((y0 + row - 1) & (S - 1)) << LGS) + xx;
+        px[k] = ld8(x + m * xs + xo + ci0 + 8 * half);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < YL; ++k) {
+      const int e = t + 256 * k;
+      py[k] = zero8();
+      if (YC % 256 == 0 || e < YC) py[k] = ld8(dy + (m0 + (e / (2 * CT))) * dys + dyo + co0 + 8 * (e % (2 * CT)));
+    }
+  };
+  f32x4 acc[NC][3][CT], bacc[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    bacc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[j][d][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = b(1.f);
+  fetch(v0);
+#pragma unroll 1
+  for (long m0 = v0; m0 < v1; m0 += BV) {
+    __syncthreads();  // the last step's reads are done
+#pragma unroll
+    for (int k = 0; k < XL; ++k) {
+      const int e = tid + 256 * k;
+      if (XC % 256 == 0 || e < XC) *(bf16x8 *)(xl + e * 8) = px[k];
+    }
+#pragma unroll
+    for (int k = 0; k < YL; ++k) {
+      const int e = tid + 256 * k, v = e / (2 * CT), c8 = e % (2 * CT);
+      if (YC % 256 == 0 || e < YC) *(bf16x8 *)(yl + (c8 >> 1) * (BV * 16) + v * 16 + (c8 & 1) * 8) = py[k];
+    }
+    __syncthreads();
+    if (m0 + BV < v1) fetch(m0 + BV);
+#pragma unroll
+    for (int q = 0; q < (NK + KW - 1) / KW; ++q) {
+      const int ks = kw * ((NK + KW - 1) / KW) + q;
+      if (NK % KW != 0 && ks >= NK) break;
+      const int row = ks * 32 / S;
+      bf16x8 a[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        const bf16 *yp = yl + c * (BV * 16) + ks * 512 + yoff;
+        a[c] = tr8(yp, yp + 64);
+        bacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], ones, bacc[c], 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const int t9 = th * NC + j;  // (dz, dy)
+        if (CT == 2 && t9 >= 9) break;
+        const bf16 *xp = xl + ((t9 / 3) * (RB + 2) + t9 % 3 + row) * (S * 16);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          // the K steps of a wave alternate over the two halves of a 64-voxel row
+          const int o0 = SEG == 2 && (q & 1) ? off[SEG - 1][0][d] : off[0][0][d];
+          const int o1 = SEG == 2 && (q & 1) ? off[SEG - 1][1][d] : off[0][1][d];
+          const bf16x8 bb = tr8(xp + o0, xp + o1);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[j][d][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], bb, acc[j][d][c], 0, 0, 0);
+        }
+      }
+    }
+  }
+  // add the voxel shares in the order kw = 0, 1, ..; the tap halves are separate.  Tile slots: CT = 1
+  // 27 taps then bias; CT = 2 15 taps of the first half, 12 (15) of the second, then bias, per co tile
+  float *sum = (float *)lds;
+#pragma unroll 1
+  for (int k = 0; k < KW; ++k) {
+    __syncthreads();
+    if (kw == k) {
+      auto add = [&](int tile, f32x4 v) {
+        float *t = sum + tile * 256 + lane * 4;
+        f32x4 o = k ? *(f32x4 *)t : f32x4{0.f, 0.f, 0.f, 0.f};
+        o += v;
+        *(f32x4 *)t = o;
+      };
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) add(((th * NC + j) * 3 + d) * CT + c, acc[j][d][c]);
+        if (th == 0) add((CT == 1 ? 27 : 30) * CT + c, bacc[c]);
+      }
+    }
+  }
+  __syncthreads();
+  // partial[chunk][co][tap][ci]
+  float *pp = partial + (long)blockIdx.x * ((long)cout * 27 * cin);
+  for (int e = tid; e < 27 * CT * 256; e += 256) {
+    const int ci = e & 15, m = (e >> 4) & 15, tc = e >> 8, tap = tc / CT, c = tc % CT;
+    if (ci0 + ci < cin)
+      pp[((long)(co0 + 16 * c + m) * 27 + tap) * cin + ci0 + ci] = sum[tc * 256 + ((m >> 2) * 16 + ci) * 4 + (m & 3)];
+  }
+  if (bpartial && blockIdx.y == 0 && tid < 16 * CT) {
+    const int c = tid >> 4, m = tid & 15;
+    bpartial[(long)blockIdx.x * cout + co0 + tid] = sum[((CT == 1 ? 27 : 30) * CT + c) * 256 + (m >> 2) * 64 + (m & 3)];
+  }
+}
+
+// out[e] = sum_p partial[p][e], deterministic; accumulate adds to out.  64 columns per workgroup, the
+// partials of a column shared by four threads (p mod 4), each with eight running sums.  One thread a
+// column left the loads a serial chain (47 us a launch on the network's layers).
+__global__ void __launch_bounds__(256) k_reduce(const float *__restrict__ partial, long np, long n, float *__restrict__ out,
+                                                int accumulate) {
+  __shared__ float red[4][64];
+  const int col = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const long e = (long)blockIdx.x * 64 + col;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (e < n) {
+    long p = q;
+    for (; p + 28 < np; p += 32)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += partial[(p + 4 * i) * n + e];
+    for (int i = 0; p < np; p += 4, ++i) s[i] += partial[p * n + e];
+  }
+  red[q][col] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  __syncthreads();
+  if (q == 0 && e < n) {
+    const float t = (red[0][col] + red[1][col]) + (red[2][col] + red[3][col]);
+    out[e] = accumulate ? out[e] + t : t;
+  }
 }
 
 // out[c] = sum_p partial[p * stride + c], c < ncols (fixed order)
@@ -551,33 +744,63 @@ extern "C" int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void
   return lg::check_launch("nn_conv3");
 }
 
-extern "C" long hgrid_nn_wgrad_chunk(long nvox) {
-  // voxels per workgroup: a multiple of 128, at most 256 chunks
-  long vc = (nvox + 255) / 256;
-  vc = (vc + WG_V - 1) / WG_V * WG_V;
-  return vc < WG_V ? WG_V : vc;
+// the cubes of k_wgrad_rows; other sides keep the tap-by-tap kernel
+static bool wgrad_by_rows(int lgS) { return lgS >= 3 && lgS <= 6; }
+
+// voxels per workgroup: a multiple of 256.  By rows, 1024 or so (256 in the smallest layers, and at
+// most 512 chunks), so that the channel tiles together fill the chip; tap by tap, at most 256 chunks
+static long wgrad_chunk(long nvox, int lgS) {
+  long n = 256;
+  if (wgrad_by_rows(lgS)) {
+    n = nvox / 1024;
+    if (n < 16) n = 16;
+    if (n > 512) n = 512;
+  }
+  const long vc = ((nvox + n - 1) / n + 255) / 256 * 256;
+  return vc;
 }
 
-extern "C" long hgrid_nn_wgrad_partials(long nvox) {
-  const long vc = hgrid_nn_wgrad_chunk(nvox);
-  return 4 * ((nvox + vc - 1) / vc);
-}
-
-extern "C" long hgrid_nn_wgrad_chunks(long nvox) {
-  const long vc = hgrid_nn_wgrad_chunk(nvox);
+extern "C" long hgrid_nn_wgrad_chunks(long nvox, int lgS) {
+  const long vc = wgrad_chunk(nvox, lgS);
   return (nvox + vc - 1) / vc;
+}
+
+extern "C" long hgrid_nn_wgrad_partials(long nvox, int lgS) {
+  return (wgrad_by_rows(lgS) ? 1 : 4) * hgrid_nn_wgrad_chunks(nvox, lgS);
+}
+
+template <int LGS>
+static void launch_wgrad_rows(dim3 grid, int ct, const bf16 *D, int dys, int dyo, const bf16 *X, int xs, int xo, int cin,
+                              long nvox, long vc, int cout, float *partial, float *bpartial) {
+  if (ct == 2)
+    hipLaunchKernelGGL((k_wgrad_rows<LGS, 2>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial);
+  else
+    hipLaunchKernelGGL((k_wgrad_rows<LGS, 1>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial);
 }
 
 extern "C" int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, const void *x, int xs, int xo, int cin,
                                     int lgS, long nvox, float *partial, float *bpartial) {
   if (cin % 8 || cin > 16 * WG_MAXT || cout % 16 || xo + cin > xs || dyo + cout > dys || nvox <= 0)
     return lg::fail("nn_conv3_wgrad: shape");
-  const long vc = hgrid_nn_wgrad_chunk(nvox);
+  const long vc = wgrad_chunk(nvox, lgS);
   const int t16 = cout / 16;
   const int ct = t16 % 2 == 0 ? 2 : 1;  // LDS: 16 CT + 16 WG_MAXT rows of WG_P bf16 stay under 64 KiB
-  dim3 grid((unsigned)((nvox + vc - 1) / vc), 27, t16 / ct);
+  const unsigned chunks = (unsigned)((nvox + vc - 1) / vc);
   auto *D = (const bf16 *)dy;
   auto *X = (const bf16 *)x;
+  if (wgrad_by_rows(lgS)) {
+    if (nvox % (1L << (3 * lgS)) || (cin % 16 && cin != 8) || ((uintptr_t)dy | (uintptr_t)x) & 15 || (dys | dyo | xs | xo) & 7)
+      return lg::fail("nn_conv3_wgrad: shape");
+    dim3 grid(chunks, (cin + 15) / 16, t16 / ct);
+    switch (lgS) {
+      case 3: launch_wgrad_rows<3>(grid, ct, D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial); break;
+      case 4: launch_wgrad_rows<4>(grid, ct, D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial); break;
+      case 5: launch_wgrad_rows<5>(grid, ct, D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial); break;
+      default: launch_wgrad_rows<6>(grid, ct, D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial); break;
+    }
+    return lg::check_launch("nn_conv3_wgrad");
+  }
+  dim3 grid(chunks, 27, t16 / ct);
   switch (ct) {
     case 2: hipLaunchKernelGGL((k_conv3_wgrad<2>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, lgS, nvox, vc, cout, partial, bpartial); break;
     default: hipLaunchKernelGGL((k_conv3_wgrad<1>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, lgS, nvox, vc, cout, partial, bpartial); break;
@@ -587,7 +810,7 @@ extern "C" int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, 
 
 extern "C" int hgrid_nn_reduce(const float *partial, long np, long n, float *out, int accumulate) {
   if (n <= 0 || np <= 0) return lg::fail("nn_reduce: shape");
-  hipLaunchKernelGGL(k_reduce, dim3(blocks(n, 256)), dim3(256), 0, lg::stream(), partial, np, n, out, accumulate);
+  hipLaunchKernelGGL(k_reduce, dim3(blocks(n, 64)), dim3(256), 0, lg::stream(), partial, np, n, out, accumulate);
   return lg::check_launch("nn_reduce");
 }
 

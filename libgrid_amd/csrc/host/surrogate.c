@@ -140,23 +140,27 @@ grid_surrogate *grid_surrogate_alloc(INT side, INT batch, REAL vscale, INT seed)
   s->vin = (float *)dalloc(sizeof(float) * nvb, "hipMalloc (surrogate input)");
   s->tgt = (float *)dalloc(sizeof(float) * nvb, "hipMalloc (surrogate target)");
   s->out = (float *)dalloc(sizeof(float) * nvb, "hipMalloc (surrogate output)");
-  /* partial-sum scratch: the largest of the weight-gradient, bias and head partials */
-  long pn = 0;
-  for (int l = 0; l < NLAYERS; ++l) {
-    const int lev = l == E1 || l == D1 ? 0 : (l == E2A || l == E2B || l == D2A || l == D2B) ? 1
-                                          : (l == E3A || l == E3B || l == D3A || l == D3B) ? 2 : 3;
-    const long nvl = lvl(s, nvb, lev);
-    const long a = hgrid_nn_wgrad_partials(nvl) * 27L * kL[l].cin * kL[l].cout;
-    const long bsum = hgrid_nn_colsum_chunks(nvl) * kL[l].cout;
-    if (a > pn) pn = a;
-    if (bsum > pn) pn = bsum;
-  }
+  /* partial-sum scratch: the largest of the weight-gradient, bias and head partials over the sizes
+   * of a minibatch */
+  long pn = 0, bn = 0;
+  for (long nb = 1; nb <= batch; ++nb)
+    for (int l = 0; l < NLAYERS; ++l) {
+      const int lev = l == E1 || l == D1 ? 0 : (l == E2A || l == E2B || l == D2A || l == D2B) ? 1
+                                            : (l == E3A || l == E3B || l == D3A || l == D3B) ? 2 : 3;
+      const long nvl = lvl(s, s->nv * nb, lev);
+      const long a = hgrid_nn_wgrad_partials(nvl, lgS - lev) * 27L * kL[l].cin * kL[l].cout;
+      const long bb = hgrid_nn_wgrad_chunks(nvl, lgS - lev) * kL[l].cout;
+      const long bsum = hgrid_nn_colsum_chunks(nvl) * kL[l].cout;
+      if (a > pn) pn = a;
+      if (bsum > pn) pn = bsum;
+      if (bb > bn) bn = bb;
+    }
   if (hgrid_nn_head_blocks(nvb) * 18 > pn) pn = hgrid_nn_head_blocks(nvb) * 18;
   s->partial_n = pn;
   s->partial = (float *)dalloc(sizeof(float) * pn, "hipMalloc (surrogate partials)");
   s->scal = (float *)dalloc(sizeof(float) * 4, "hipMalloc (surrogate scalars)");
   s->clip_scratch = (double *)dalloc(sizeof(double) * 512, "hipMalloc (clip scratch)");
-  s->bpartial = (float *)dalloc(sizeof(float) * (size_t)(hgrid_nn_wgrad_chunks(nvb) * 192), "hipMalloc (bias partials)");
+  s->bpartial = (float *)dalloc(sizeof(float) * (size_t)bn, "hipMalloc (bias partials)");
   return s;
 }
 
@@ -233,8 +237,8 @@ static void wgrad(grid_surrogate *s, int l, const void *dy, const void *x, int x
   const int ci = kL[l].cin, co = kL[l].cout;
   lg_hip(hgrid_nn_conv3_wgrad(dy, co, 0, co, x, xs, xo, ci, s->lgS - lev, nvl, s->partial, s->bpartial),
          "nn_conv3_wgrad");
-  lg_hip(hgrid_nn_reduce(s->partial, hgrid_nn_wgrad_partials(nvl), 27L * ci * co, s->g + s->off_w[l], 0), "nn_reduce");
-  lg_hip(hgrid_nn_reduce(s->bpartial, hgrid_nn_wgrad_chunks(nvl), co, s->g + s->off_b[l], 0), "nn_reduce (bias)");
+  lg_hip(hgrid_nn_reduce(s->partial, hgrid_nn_wgrad_partials(nvl, s->lgS - lev), 27L * ci * co, s->g + s->off_w[l], 0), "nn_reduce");
+  lg_hip(hgrid_nn_reduce(s->bpartial, hgrid_nn_wgrad_chunks(nvl, s->lgS - lev), co, s->g + s->off_b[l], 0), "nn_reduce (bias)");
 }
 
 /* data gradient of layer l: dx = conv^T(dy), optionally times (act > 0) */

@@ -140,3 +140,52 @@ def test_symgather_matches_numpy(lg):
     finally:
         lg.hgrid_free(d_src)
         lg.hgrid_free(d_dst)
+
+
+@pytest.mark.parametrize("S,cin,cout", [(64, 8, 16), (64, 48, 16), (64, 16, 32), (32, 48, 16), (32, 96, 32), (16, 32, 64),
+                                        (16, 16, 16), (8, 64, 32), (8, 8, 16)])
+def test_weight_gradient_kernel(lg, S, cin, cout):
+    """dW and the bias gradient of one convolution over two samples, for every cube side and tile count
+    of the row kernel, against float64 numpy.  Inputs are multiples of 1/64 that BF16 holds, so only
+    the FP32 sums round: chains of at most a few thousand additions, 1e-5 relative at most."""
+    print(f"[case] weight gradient S {S} cin {cin} cout {cout}", flush=True)
+    rng = np.random.default_rng(S + cin + cout)
+    n, lgS = 2 * S**3, S.bit_length() - 1
+    xs, xo, ys, yo = cin + 24, 16, cout + 8, 8
+    X = rng.integers(-127, 128, (n, xs)) / 64.0
+    dY = rng.integers(-127, 128, (n, ys)) / 64.0
+
+    def up(a):
+        h = (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        p = C.c_void_p()
+        assert lg.hgrid_malloc(C.byref(p), h.nbytes) == 0
+        assert lg.hgrid_memcpy_h2d(p, h.ctypes.data, h.nbytes) == 0
+        return p
+
+    f = lg.hgrid_nn_conv3_wgrad
+    f.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_long, C.c_void_p,
+                  C.c_void_p]
+    for name in ("hgrid_nn_wgrad_partials", "hgrid_nn_wgrad_chunks"):
+        getattr(lg, name).argtypes = [C.c_long, C.c_int]
+        getattr(lg, name).restype = C.c_long
+    lg.hgrid_nn_reduce.argtypes = [C.c_void_p, C.c_long, C.c_long, C.c_void_p, C.c_int]
+    m = 27 * cin * cout
+    nparts, nchunks = lg.hgrid_nn_wgrad_partials(n, lgS), lg.hgrid_nn_wgrad_chunks(n, lgS)
+    px, py, part, bpart, out = up(X), up(dY), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    for p, count in ((part, nparts * m), (bpart, nchunks * cout), (out, m + cout)):
+        assert lg.hgrid_malloc(C.byref(p), 4 * count) == 0
+    assert f(py, ys, yo, cout, px, xs, xo, cin, lgS, n, part, bpart) == 0
+    assert lg.hgrid_nn_reduce(part, nparts, m, out, 0) == 0
+    assert lg.hgrid_nn_reduce(bpart, nchunks, cout, out.value + 4 * m, 0) == 0
+    got = np.empty(m + cout, dtype=np.float32)
+    assert lg.hgrid_memcpy_d2h(got.ctypes.data, out, got.nbytes) == 0
+    for p in (px, py, part, bpart, out):
+        lg.hgrid_free(p)
+    x5 = X[:, xo:xo + cin].reshape(2, S, S, S, cin)
+    y2 = dY[:, yo:yo + cout]
+    ref = np.empty((cout, 27, cin))
+    for t in range(27):
+        d = (t // 9 - 1, t // 3 % 3 - 1, t % 3 - 1)
+        ref[:, t] = y2.T @ np.roll(x5, [-k for k in d], (1, 2, 3)).reshape(n, cin)
+    assert np.linalg.norm(got[:m] - ref.ravel()) / np.linalg.norm(ref) < 1e-5
+    assert np.linalg.norm(got[m:] - y2.sum(0)) / np.linalg.norm(y2.sum(0)) < 1e-5
