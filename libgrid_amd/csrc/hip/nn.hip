@@ -42,64 +42,86 @@ __device__ __forceinline__ long nbr(long bz, int z, int y, int x, int t, int lgS
 // ---- convolution: implicit GEMM, M = voxels, N = output channels, K = 27 Cin ----------------
 // Each wave computes MT x NTL tiles of 16 x 16; a workgroup is 4 waves over consecutive voxels.
 // With reflected, transposed weights (k_wprep) the same kernel computes the data gradient.
-template <int MT, int NTL>
+//
+// Bound by the loads: a chain of latencies in small grids (DEPTH steps of operands are in flight), the
+// address units' 64 bytes a cycle in large ones.  The addresses cost little: a table in LDS gives each
+// chunk's tap as packed coordinate offsets, and the wrapped neighbour is formed field by field in one
+// add and two xors (below).
+constexpr int CONV_CH = 27 * 24 + 12;  // chunks of the largest Cin (192), and past the end
+
+template <int MT, int NTL, int DEPTH>
 __global__ void __launch_bounds__(256) k_conv3(const bf16 *__restrict__ x, int xs, int xo, int cin,
                                                const bf16 *__restrict__ w, const float *__restrict__ bias,
                                                bf16 *__restrict__ y, int ys, int yo, const bf16 *__restrict__ mask,
                                                int mks, int mko, int lgS, long nvox, int relu) {
+  __shared__ int2 chunk[CONV_CH];  // {packed offsets of the tap, first channel or -1 past the end}
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, r = lane & 15;
   const long m0 = ((long)blockIdx.x * 4 + wave) * (16 * MT);
   const int co0 = blockIdx.y * (16 * NTL);
   const int msk = (1 << lgS) - 1;
-  const int nch = 27 * (cin >> 3);
-  long vb[MT];
-  int vz[MT], vy[MT], vx[MT];
+  const int cpt = cin >> 3, nch = 27 * cpt;
+  for (int c = threadIdx.x; c < nch + 12; c += 256) {
+    const int t = c / cpt, dz = t / 9 + msk, dy = (t / 3) % 3 + msk, dx = t % 3 + msk;  // -1 .. 1 mod S
+    chunk[c] = c < nch ? make_int2(((dz & msk) << (2 * lgS)) | ((dy & msk) << lgS) | (dx & msk), (c - t * cpt) * 8)
+                       : make_int2(0, -1);
+  }
+  __syncthreads();
+  // voxel index in the sample = z | y | x, lgS bits each.  With TOP the top bit of each field,
+  // (m + d) mod S field by field = ((m & ~TOP) + (d & ~TOP)) ^ ((m ^ d) & TOP): no carry leaves a field
+  const unsigned top = (1u << (lgS - 1)) | (1u << (2 * lgS - 1)) | (1u << (3 * lgS - 1)), field = (1u << (3 * lgS)) - 1;
+  const bf16 *base[MT];
+  unsigned low[MT], high[MT];
   bool vok[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const long m = m0 + 16 * mt + r;
     vok[mt] = m < nvox;
     const long mm = vok[mt] ? m : 0;
-    vx[mt] = (int)(mm & msk);
-    vy[mt] = (int)((mm >> lgS) & msk);
-    vz[mt] = (int)((mm >> (2 * lgS)) & msk);
-    vb[mt] = (mm >> (3 * lgS)) << (3 * lgS);
+    low[mt] = (unsigned)mm & field & ~top;
+    high[mt] = (unsigned)mm & top;
+    base[mt] = x + ((mm >> (3 * lgS)) << (3 * lgS)) * xs + xo;
   }
+  const bf16 *wl = w + (long)(co0 + r) * 27 * cin + 8 * g;
+  const long wtile = 16L * 27 * cin;
   f32x4 acc[MT][NTL];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int j = 0; j < NTL; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // chunk kc + g of every step: (tap, channel block cb)
-  int tap = 0, cb = 8 * g;
-  while (cb >= cin) {
-    cb -= cin;
-    ++tap;
-  }
-  const long wrow = 27L * cin;
-#pragma unroll 1
-  for (int kc = 0; kc < nch; kc += 4) {
-    const bool cok = tap < 27;
-    bf16x8 a[MT], bw[NTL];
+  bf16x8 a[DEPTH][MT], bw[DEPTH][NTL];
+  auto fetch = [&](int kc, bf16x8(&av)[MT], bf16x8(&bv)[NTL]) {
+    const int2 ch = chunk[kc + g];
+    const bool cok = ch.y >= 0;
+    const unsigned dl = (unsigned)ch.x & ~top, dh = (unsigned)ch.x & top;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      a[mt] = zero8();
-      if (cok && vok[mt]) a[mt] = ld8(x + nbr(vb[mt], vz[mt], vy[mt], vx[mt], tap, lgS) * xs + xo + cb);
+      av[mt] = zero8();
+      if (cok && vok[mt]) av[mt] = ld8(base[mt] + (long)((low[mt] + dl) ^ high[mt] ^ dh) * xs + ch.y);
     }
 #pragma unroll
     for (int j = 0; j < NTL; ++j) {
-      bw[j] = zero8();
-      if (cok) bw[j] = ld8(w + (long)(co0 + 16 * j + r) * wrow + tap * cin + cb);
+      bv[j] = zero8();
+      if (cok) bv[j] = ld8(wl + j * wtile + 8L * kc);
     }
+  };
+  auto products = [&](const bf16x8(&av)[MT], const bf16x8(&bv)[NTL]) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int j = 0; j < NTL; ++j) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bw[j], acc[mt][j], 0, 0, 0);
-    cb += 32;
-    while (cb >= cin) {
-      cb -= cin;
-      ++tap;
+      for (int j = 0; j < NTL; ++j) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt], bv[j], acc[mt][j], 0, 0, 0);
+  };
+  // step k's operands are fetched DEPTH - 1 steps ahead into slot k mod DEPTH; chunks past the end are
+  // zeros and add nothing
+#pragma unroll
+  for (int k = 0; k < DEPTH - 1; ++k) fetch(4 * k, a[k], bw[k]);
+#pragma unroll 1
+  for (int kc = 0; kc < nch; kc += 4 * DEPTH) {
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) {
+      if (k && kc + 4 * k >= nch) break;
+      fetch(kc + 4 * (k + DEPTH - 1), a[(k + DEPTH - 1) % DEPTH], bw[(k + DEPTH - 1) % DEPTH]);
+      products(a[k], bw[k]);
     }
   }
 #pragma unroll
@@ -727,20 +749,28 @@ extern "C" int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void
       nvox <= 0 || nvox % (1L << (3 * lgS)))
     return lg::fail("nn_conv3: shape");
   if (((uintptr_t)x | (uintptr_t)w) & 15) return lg::fail("nn_conv3: operands must be 16-byte aligned");
+  if (cin > 192 || lgS > 10) return lg::fail("nn_conv3: shape");
+  // tiles of 2 or 4 voxel groups x up to 4 channel groups share operands; where that leaves fewer than
+  // 1024 waves (four per CU) single tiles make more of them, and the operands are fetched two steps
+  // ahead, which larger grids cannot afford in registers (48 -> 16 channels, 8 x 64^3: 460 us without,
+  // but 32 -> 32 at 8 x 32^3 60 against 85 us with; 128 -> 128 at 8^3: 57 -> 28 us in single tiles)
   const int t16 = cout / 16;
-  const int ntl = t16 % 4 == 0 ? 4 : t16 % 3 == 0 ? 3 : t16 % 2 == 0 ? 2 : 1;
-  const int mt = ntl == 1 ? 4 : 2;
+  int ntl = t16 % 4 == 0 ? 4 : t16 % 3 == 0 ? 3 : t16 % 2 == 0 ? 2 : 1;
+  int mt = ntl == 1 ? 4 : 2;
+  if (nvox / (16 * mt) * (t16 / ntl) < 1024) ntl = mt = 1;
   dim3 grid(blocks(nvox, 64 * mt), t16 / ntl);
   auto *X = (const bf16 *)x;
   auto *W = (const bf16 *)w;
   auto *Y = (bf16 *)y;
   auto *M = (const bf16 *)mask;
-  switch (ntl) {
-    case 4: hipLaunchKernelGGL((k_conv3<2, 4>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu); break;
-    case 3: hipLaunchKernelGGL((k_conv3<2, 3>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu); break;
-    case 2: hipLaunchKernelGGL((k_conv3<2, 2>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu); break;
-    default: hipLaunchKernelGGL((k_conv3<4, 1>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu); break;
-  }
+#define LG_CONV(mtv, ntlv, depth) \
+  hipLaunchKernelGGL((k_conv3<mtv, ntlv, depth>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu)
+  if (ntl == 4) LG_CONV(2, 4, 1);
+  else if (ntl == 3) LG_CONV(2, 3, 1);
+  else if (ntl == 2) LG_CONV(2, 2, 1);
+  else if (mt == 4) LG_CONV(4, 1, 1);
+  else LG_CONV(1, 1, 3);
+#undef LG_CONV
   return lg::check_launch("nn_conv3");
 }
 
