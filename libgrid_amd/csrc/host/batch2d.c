@@ -153,7 +153,6 @@ static void b2d_pack(b2d_batch *b, INT ns, wf **gwf, rgrid **pot, REAL dt, REAL 
   if (b->hist_len > 0)
     lg_hip(hgrid_malloc((void **)&b->hist, sizeof(double) * (size_t)(b->hist_len * ns)), "hipMalloc (batch history)");
   b->hjobs = (hgrid_b2d_job *)calloc(ns, sizeof(hgrid_b2d_job));
-  long toff = 0;
   /* queue order: largest grids first (longest solves start early) */
   long *order = (long *)malloc(sizeof(long) * 2 * ns);
   for (INT i = 0; i < ns; ++i) {
@@ -161,13 +160,23 @@ static void b2d_pack(b2d_batch *b, INT ns, wf **gwf, rgrid **pot, REAL dt, REAL 
     order[2 * i + 1] = i;
   }
   qsort(order, ns, 2 * sizeof(long), cmp_desc);
+  long *tab_off = (long *)malloc(sizeof(long) * (size_t)(ns + 1));
+  if (!tab_off) lg_fatal("out of host memory (batched solves)");
+  tab_off[0] = 0;
+  for (INT r = 0; r < ns; ++r) {
+    INT i = order[2 * r + 1];
+    cgrid_host_sync(gwf[i]->grid);
+    rgrid_host_sync(pot[i]);
+    tab_off[r + 1] = tab_off[r] + gwf[i]->grid->ny * (4 + 4 + 8 + 8);
+  }
+  /* the problems are packed side by side: an exponential a point, the largest share of a short call
+   * (48 problems, 128 steps: 10 of 18 ms on one thread) */
+#pragma omp parallel for schedule(dynamic, 1)
   for (INT r = 0; r < ns; ++r) {
     INT i = order[2 * r + 1];
     cgrid *g = gwf[i]->grid;
     rgrid *v = pot[i];
-    const long n = g->ny, nn = n * n, o = b->off[i];
-    cgrid_host_sync(g);
-    rgrid_host_sync(v);
+    const long n = g->ny, nn = n * n, o = b->off[i], toff = tab_off[r];
     for (long k = 0; k < nn; ++k) {
       hpsi[2 * (o + k)] = (float)creal(g->value[k]);
       hpsi[2 * (o + k) + 1] = (float)cimag(g->value[k]);
@@ -214,8 +223,8 @@ static void b2d_pack(b2d_batch *b, INT ns, wf **gwf, rgrid **pot, REAL dt, REAL 
     j->out = b->out + HGRID_B2D_NOUT * i;
     j->hist_len = (int)b->hist_len;
     j->hist = b->hist ? b->hist + b->hist_len * i : NULL;
-    toff += n * (4 + 4 + 8 + 8);
   }
+  free(tab_off);
   free(order);
   lg_hip(hgrid_memcpy_h2d(b->psi_pool, hpsi, sizeof(float) * 2 * total), "hipMemcpy (batch psi)");
   lg_hip(hgrid_memcpy_h2d(b->pv_pool, hpv, sizeof(float) * total), "hipMemcpy (batch pv)");
@@ -367,10 +376,14 @@ REAL grid_wf_batch2d_relax(INT nsolves, wf **gwf, rgrid **potential, REAL dt, RE
   }
   float *hpsi = (float *)malloc(sizeof(float) * 2 * b.total);
   lg_hip(hgrid_memcpy_d2h(hpsi, b.psi_pool, sizeof(float) * 2 * b.total), "hipMemcpy (batch psi)");
+#pragma omp parallel for schedule(dynamic, 1)
   for (INT i = 0; i < nsolves; ++i) {
     cgrid *g = gwf[i]->grid;
     const long nn = g->ny * g->nz, o = b.off[i];
     for (long k = 0; k < nn; ++k) g->value[k] = (double)hpsi[2 * (o + k)] + I * (double)hpsi[2 * (o + k) + 1];
+  }
+  for (INT i = 0; i < nsolves; ++i) {
+    cgrid *g = gwf[i]->grid;
     cgrid_host_modified(g);
     if (out[HGRID_B2D_NOUT * i + 2] == -2.0 || !isfinite(out[HGRID_B2D_NOUT * i]))
       lg_fatal("batched relaxation: solve %ld (%ld x %ld) diverged: non-finite energy", (long)i, (long)g->ny, (long)g->nz);

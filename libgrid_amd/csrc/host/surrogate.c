@@ -308,15 +308,27 @@ static void adam_step(grid_surrogate *s, double lr) {
   refresh_weights(s);
 }
 
+/* the interface's doubles to the network's floats and back, by all host threads where there are enough
+ * of them (one 64^3 sample is done before the threads are awake) */
+static void narrow(float *dst, const REAL *src, long n) {
+#pragma omp parallel for schedule(static) if (n > (1L << 20))
+  for (long i = 0; i < n; ++i) dst[i] = (float)src[i];
+}
+
+static void widen(REAL *dst, const float *src, long n) {
+#pragma omp parallel for schedule(static) if (n > (1L << 20))
+  for (long i = 0; i < n; ++i) dst[i] = src[i];
+}
+
 static void upload_batch(grid_surrogate *s, long nb, const REAL *pot, const REAL *target) {
   const long n = s->nv * nb;
   if (n <= 0) return;
   float *h = (float *)malloc(sizeof(float) * (size_t)n);
   if (!h) lg_fatal("out of host memory (surrogate batch)");
-  for (long i = 0; i < n; ++i) h[i] = (float)pot[i];
+  narrow(h, pot, n);
   lg_hip(hgrid_memcpy_h2d(s->vin, h, sizeof(float) * n), "hipMemcpy (surrogate input)");
   if (target) {
-    for (long i = 0; i < n; ++i) h[i] = (float)target[i];
+    narrow(h, target, n);
     lg_hip(hgrid_memcpy_h2d(s->tgt, h, sizeof(float) * n), "hipMemcpy (surrogate target)");
   }
   free(h);
@@ -330,7 +342,7 @@ REAL grid_surrogate_gradient(grid_surrogate *s, INT nb, const REAL *pot, const R
   if (grad) {
     float *h = (float *)malloc(sizeof(float) * s->np);
     lg_hip(hgrid_memcpy_d2h(h, s->g, sizeof(float) * s->np), "hipMemcpy (grads)");
-    for (long i = 0; i < s->np; ++i) grad[i] = h[i];
+    widen(grad, h, s->np);
     free(h);
   }
   return loss;
@@ -343,7 +355,7 @@ void grid_surrogate_predict(grid_surrogate *s, INT n, const REAL *pot, REAL *amp
     upload_batch(s, nb, pot + i0 * s->nv, NULL);
     forward(s, s->nv * nb);
     lg_hip(hgrid_memcpy_d2h(h, s->out, sizeof(float) * s->nv * nb), "hipMemcpy (surrogate output)");
-    for (long i = 0; i < s->nv * nb; ++i) amp[i0 * s->nv + i] = h[i];
+    widen(amp + i0 * s->nv, h, s->nv * nb);
   }
   free(h);
 }
