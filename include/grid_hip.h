@@ -150,6 +150,7 @@ int hgrid_fft_supported(long n);
  * A 2-D grid has no x: its h takes x's place (flat). */
 typedef struct hgrid_tile {
   void *psi;             /* device array (complex, precision prec), transformed in place */
+  void *out;             /* HGRID_TILE_POT: another array for the result (NULL: in place) */
   int prec;              /* HGRID_C128 / HGRID_C64 */
   long n0, n1, n2;       /* squeezed shape; n2 is contiguous */
   /* filled in by hgrid_tile_plan */
@@ -163,6 +164,11 @@ typedef struct hgrid_tile {
                           * B: PRESCALE, PRE_VEFF, PRE_RED, POT_NOFFT1, POT_NOFFT2, POST_RED */
   const void *twx, *twl, *twz, *twy;  /* exp(-2 pi i m / n) of x (2-D: h), rows, n2 and n1 */
   const double *scale;
+  /* A, PRESCALE with scale NULL: the factor sqrt(norm_target / (norm_dv sum)), sum the total of
+   * norm_count partials that the pass before wrote */
+  const double *norm_partials;
+  long norm_count;
+  double norm_target, norm_dv;
   double post;           /* A: real factor applied to the input */
   const void *ktab_0, *ktab_1, *ktab_2;   /* kinetic tables (double2) per axis, natural order */
   const double *k2_0, *k2_1;              /* |k|^2 for MID_KRED; z's is formed from k2_dk */

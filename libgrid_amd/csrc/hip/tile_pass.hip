@@ -98,6 +98,7 @@ extern "C" int hgrid_tile_pass(const hgrid_tile *t, int pass) {
   if (!t || !hgrid_tile_plan(t->prec, t->n0, t->n1, t->n2, &shape) || shape.rows != t->rows || shape.nh != t->nh ||
       shape.flat != t->flat || shape.sx != t->sx || shape.sh != t->sh)
     return -1;
+  if ((t->flags & HGRID_PF_PRESCALE) && !t->scale && (pass != HGRID_TILE_KINETIC || !t->norm_partials || t->norm_count < 1)) return -1;
   const bool f64 = t->prec == HGRID_C128;
   switch (pass) {
     case HGRID_TILE_KINETIC: return f64 ? lg::tile::launch_kinetic_f64(t) : lg::tile::launch_kinetic_f32(t);

@@ -375,7 +375,7 @@ template <int NT> __device__ __forceinline__ void reduce_partials(double (&acc)[
 
 // Waves per SIMD asked of the register allocator: 128 VGPRs for tiles of 16 FP64 or 32 FP32 values
 // per thread (two workgroups of 512 threads per CU).
-template <typename C, int R> constexpr int waves() { return sizeof(C) == 16 ? (R <= 16 ? 4 : 2) : R >= 24 ? 3 : 5; }
+template <typename C, int R> constexpr int waves() { return sizeof(C) == 16 ? (R <= 16 ? 4 : 3) : R >= 24 ? 3 : 5; }
 // FP32 data with real factors multiplies in FP64 and needs more
 template <typename C, int R, bool REALK> constexpr int waves_a() { return sizeof(C) == 8 && REALK ? (R >= 24 ? 3 : 4) : waves<C, R>(); }
 
@@ -398,6 +398,30 @@ __attribute__((amdgpu_waves_per_eu(waves_a<C, GeomA<C, LZ, B>::R, REALK>(), 8)))
   AZ::fill(tabz, tid, (const C *)a.twz);
   AY::fill(taby, tid, (const C *)a.twl);
   const auto rio = make_rsrc((const C *)a.psi + (long)blockIdx.x * T, (unsigned long)T * CS);
+  C scale = mk<C>((Rl)1, (Rl)0);
+  if ((fl & HGRID_PF_PRESCALE) && a.scale) {
+    scale = mk<C>((Rl)a.scale[0], (Rl)a.scale[1]);
+  } else if (fl & HGRID_PF_PRESCALE) {
+    // the renormalisation of a relaxation step, from the partial sums of the pass before: every
+    // workgroup adds them in the same order, which saves a launch a step (64^3 FP32: 3.2 of 15 us)
+    constexpr int WHOLE = NT % 64 == 0, NS = WHOLE ? NT / 64 : NT;
+    __shared__ double sums[NS];
+    double s = 0.0;
+    for (long i = tid; i < a.norm_count; i += NT) s += a.norm_partials[i];
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    }
+    if (!WHOLE || tid % 64 == 0) sums[WHOLE ? tid / 64 : tid] = s;
+    __syncthreads();
+    s = 0.0;
+    for (int w = 0; w < NS; ++w) s += sums[w];
+    // the same in all lanes: held once, not per lane
+    const double f = sqrt(a.norm_target / (a.norm_dv * s));
+    const unsigned long long fb = __double_as_longlong(f);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)fb), hi = __builtin_amdgcn_readfirstlane((int)(fb >> 32));
+    scale.x = (Rl)__longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+  }
   C v[R];
 #pragma unroll
   for (int u = 0; u < R / Y0::r; ++u) {
@@ -407,9 +431,8 @@ __attribute__((amdgpu_waves_per_eu(waves_a<C, GeomA<C, LZ, B>::R, REALK>(), 8)))
   }
   double acc[HGRID_RED_NCHAN] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (fl & HGRID_PF_PRESCALE) {
-    const C s = mk<C>((Rl)a.scale[0], (Rl)a.scale[1]);
 #pragma unroll
-    for (int j = 0; j < R; ++j) v[j] = cmul(v[j], s);
+    for (int j = 0; j < R; ++j) v[j] = cmul(v[j], scale);
   }
   if (a.post != 1.0) {
     const Rl post = (Rl)a.post;
@@ -551,11 +574,12 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   };
   auto store = [&](auto stage, unsigned step, auto &&at) {
     using S = decltype(stage);
+    const auto rout = make_rsrc(KIND == TPOT && a.out ? a.out : a.psi, ntot * CS);
 #pragma unroll
     for (int u = 0; u < R / S::r; ++u) {
       const unsigned e = at(tid, u);
 #pragma unroll
-      for (int i = 0; i < S::r; ++i) bstore<C>(v[u * S::r + i], rio, e * CS, (unsigned)i * step * CS);
+      for (int i = 0; i < S::r; ++i) bstore<C>(v[u * S::r + i], rout, e * CS, (unsigned)i * step * CS);
     }
   };
   auto real_element = [&](int t, int u) { return element(SV::lin(t, u)); };
@@ -571,24 +595,30 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
         for (int u = 0; u < R / A; ++u) v[u * A + i] = cmul(v[u * A + i], w);
       }
     } else {
+      // by scalar steps from one address: one for each value, kept from the inverse side for the
+      // forward one, would spill
+      const auto rtw = make_rsrc(tw, (unsigned long)a.n1 * CS);
 #pragma unroll
       for (int u = 0; u < R / XL::r; ++u) {
-        const int k = frequency(tid, u);
+        const unsigned k = l * (unsigned)frequency(tid, u) * CS;
 #pragma unroll
-        for (int i = 0; i < XL::r; ++i) v[u * XL::r + i] = cmul(v[u * XL::r + i], tw[(int)l * (k + XH * i)]);
+        for (int i = 0; i < XL::r; ++i) {
+          v[u * XL::r + i] = cmul(v[u * XL::r + i], bload<C>(rtw, k, l * (unsigned)(XH * i) * CS));
+        }
       }
     }
   };
   const bool skip1 = (KIND == TPRE || KIND == TPOT) && (fl & HGRID_PF_POT_NOFFT1);
   const bool skip2 = KIND == TPRE || (KIND == TPOT && (fl & HGRID_PF_POT_NOFFT2));
+  C scale = mk<C>((Rl)1, (Rl)0);
+  if (fl & HGRID_PF_PRESCALE) scale = mk<C>((Rl)a.scale[0], (Rl)a.scale[1]);
   if (skip1) load(SV{}, stepv, real_element);
   else load(XL{}, stepl, form_element);
   if constexpr (AX::TABLE) tile_sync<NT>();
   if constexpr (KIND == TPRE || KIND == TPOT) {
     if (fl & HGRID_PF_PRESCALE) {
-      const C s = mk<C>((Rl)a.scale[0], (Rl)a.scale[1]);
 #pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = cmul(v[j], s);
+      for (int j = 0; j < R; ++j) v[j] = cmul(v[j], scale);
     }
   }
   double acc[HGRID_RED_NCHAN] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -623,6 +653,12 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
       dft_items<C, R, A>(v);
     }
     conj_all(v);
+    // without h no barrier follows, and the compiler would move the last digit's arithmetic behind the
+    // loads of the potential, its twiddles waiting in scratch (96 x 1 in FP64: 81 registers)
+    if constexpr (A == 1) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) asm volatile("" : "+v"(v[j].x), "+v"(v[j].y));
+    }
   } else {
     load_potential();
   }
@@ -647,22 +683,30 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
     return;
   } else if constexpr (KIND == TPOT) {
     if (a.pot) {
+      // four values ahead of the factors that use them
       const auto rpot = make_rsrc(a.pot, ntot * CS);
+      constexpr int AHEAD = R % 4 == 0 ? 4 : R;
+      C p[2][AHEAD];
+      auto fetch = [&](int j0, C(&q)[AHEAD]) {
 #pragma unroll
-      for (int u = 0; u < R / SV::r; ++u) {
-        const unsigned e = real_element(tid, u);
-        C p[SV::r];
-#pragma unroll
-        for (int i = 0; i < SV::r; ++i) p[i] = bload<C>(rpot, e * CS, (unsigned)i * stepv * CS);
-#pragma unroll
-        for (int i0 = 0; i0 < SV::r; i0 += GROUP) {
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = i0; i < (i0 + GROUP < SV::r ? i0 + GROUP : SV::r); ++i)
-            v[u * SV::r + i] = cmul(v[u * SV::r + i], phase_factor<C>(a.c_re, a.c_im, a.cons + (double)p[i].x, (double)p[i].y));
+        for (int j = 0; j < AHEAD; ++j) {
+          const int u = (j0 + j) / SV::r, i = (j0 + j) % SV::r;
+          q[j] = bload<C>(rpot, real_element(tid, u) * CS, (unsigned)i * stepv * CS);
         }
+      };
+      fetch(0, p[0]);
+#pragma unroll
+      for (int j0 = 0; j0 < R; j0 += AHEAD) {
         __builtin_amdgcn_sched_barrier(0);
+        if (j0 + AHEAD < R) fetch(j0 + AHEAD, p[(j0 / AHEAD + 1) % 2]);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+          if (j % GROUP == 0) __builtin_amdgcn_sched_barrier(0);
+          const C q = p[(j0 / AHEAD) % 2][j];
+          v[j0 + j] = cmul(v[j0 + j], phase_factor<C>(a.c_re, a.c_im, a.cons + (double)q.x, (double)q.y));
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   } else {
     auto factors = [&](auto &&apply) {

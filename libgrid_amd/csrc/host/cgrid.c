@@ -164,25 +164,43 @@ static void download(cgrid *g) {
   d->valid |= GV_HOST;
 }
 
-/* Transform a state left transformed by a fused step back to real space (unnormalised inverse:
- * the step's kinetic factor already carried 1/N). */
-void lg_c_materialize(cgrid *g) {
+/* The inverse transform that brings a state left transformed by a fused step back to real space
+ * (unnormalised: the step's kinetic factor already carried 1/N), from its array into out, which may
+ * be the same; scale: a device factor to apply, or NULL. */
+static void inverse_into(cgrid *g, void *out, const double *scale) {
   grid_dev *d = g->dev;
   if (d->kpend) lg_fatal("internal: a merged relaxation batch left its state between kinetic half-steps");
-  if (!d->zpend) return;
   lg_shape s;
   lg_squeeze(g->nx, g->ny, g->nz, &s);
   if (d->zpend == 2) {
     hgrid_tile t;
     if (!lg_tile_init(&t, &s, d->prec, d->d)) lg_fatal("internal: a grid in tile form that tile passes do not cover");
-    t.flags = HGRID_PF_POT_NOFFT2;
+    t.out = out;
+    t.flags = HGRID_PF_POT_NOFFT2 | (scale ? HGRID_PF_PRESCALE : 0);
+    t.scale = scale;
     lg_run_tile(&t, HGRID_TILE_POT);
   } else {
     hgrid_pass p;
-    lg_pass_init(&p, &s, d->prec, d->d, d->d, 2);
+    lg_pass_init(&p, &s, d->prec, d->d, out, 2);
     p.dir1 = +1;
+    if (scale) {
+      p.flags |= HGRID_PF_PRESCALE;
+      p.scale = scale;
+    }
     lg_run_pass(&p);
   }
+}
+
+static void scale_applied(grid_dev *d) {
+  lg_hip(hgrid_scalar_set(d->dscal + GS_SCALE, 1.0, 0.0), "scalar_set");
+  d->pending = 0;
+}
+
+void lg_c_materialize(cgrid *g) {
+  grid_dev *d = g->dev;
+  if (d->kpend) lg_fatal("internal: a merged relaxation batch left its state between kinetic half-steps");
+  if (!d->zpend) return;
+  inverse_into(g, d->d, NULL);
   d->zpend = 0;
 }
 
@@ -197,6 +215,14 @@ void *lg_c_raw(cgrid *g, const double **scale) {
 void *lg_c_in(cgrid *g, const double **scale) {
   grid_dev *d = lg_cdev(g);
   if (!(d->valid & GV_DEV)) upload(g);
+  if (!scale && d->pending && d->zpend) {
+    /* the inverse transform applies the pending scale */
+    inverse_into(g, d->d, d->dscal + GS_SCALE);
+    d->zpend = 0;
+    scale_applied(d);
+    d->valid = GV_DEV;
+    return d->d;
+  }
   lg_c_materialize(g);
   if (scale) *scale = d->pending ? d->dscal + GS_SCALE : NULL;
   else if (d->pending) lg_c_flush(g);
@@ -262,16 +288,14 @@ void lg_c_flush(cgrid *g) {
   grid_dev *d = g->dev;
   if (!d->pending) return;
   lg_hip(hgrid_cscale(d->d, d->prec, (long)d->n, 1.0, 0.0, d->dscal + GS_SCALE), "cscale");
-  lg_hip(hgrid_scalar_set(d->dscal + GS_SCALE, 1.0, 0.0), "scalar_set");
-  d->pending = 0;
+  scale_applied(d);
   d->valid = GV_DEV;
 }
 
 void lg_c_host_sync(cgrid *g) {
   grid_dev *d = g->dev;
   if (d->valid & GV_HOST) return;
-  lg_c_materialize(g);
-  lg_c_flush(g);
+  lg_c_in_flushed(g);
   download(g);
 }
 
@@ -402,8 +426,18 @@ void cgrid_copy(cgrid *dst, cgrid *src) {
   dst->ky0 = src->ky0;
   dst->kz0 = src->kz0;
   if (dst == src) return;
+  grid_dev *dd = dst->dev, *sd = src->dev;
+  if (sd->zpend && (sd->valid & GV_DEV) && dd->prec == sd->prec) {
+    /* a state between fused steps: its inverse transform goes straight into the copy, with the pending
+     * scale, and the state stays as the next step takes it (a snapshot then costs one sweep, not
+     * the transform, the scale, the copy and the way back into the step's form) */
+    lg_cdev(src);
+    void *o = lg_c_out(dst);
+    inverse_into(src, o, sd->pending ? sd->dscal + GS_SCALE : NULL);
+    lg_c_written(dst, 1);
+    return;
+  }
   void *s = lg_c_in_flushed(src);
-  grid_dev *dd = dst->dev;
   if (lg_prec_size(dd->prec) != lg_prec_size(src->dev->prec)) {
     /* copy between FP64 and FP32 storage */
     void *o = lg_c_out(dst);

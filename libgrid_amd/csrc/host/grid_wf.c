@@ -341,10 +341,19 @@ static int tile_step(wf *gwf, const step_args *sa) {
   const int veff = sa->gpe && sa->g != 0.0;
   if (veff && !d->rho) lg_hip(hgrid_malloc((void **)&d->rho, d->n * sizeof(double)), "hipMalloc (density)");
   const long nbA = base.blocks_a, nbB = base.blocks_b, nbP = nbA > nbB ? nbA : nbB;
-  double *partB = lg_partials(HGRID_RED_NCHAN * (nbB + nbA + nbP));
+  /* the sums handed on within a merged batch have a place of their own: the A-pass that reads them
+   * writes others */
+  double *partB = lg_partials(HGRID_RED_NCHAN * (nbB + nbA + nbP + nbB));
   double *partK = partB + HGRID_RED_NCHAN * nbB, *partP = partK + HGRID_RED_NCHAN * nbA;
+  double *partH = partP + HGRID_RED_NCHAN * nbP;
   const double *pend = scale; /* the pending scale, until a pass that stores has applied it */
   double post = 1.0;
+  /* the steps of a merged batch hand the norm's partial sums to the next one, which nothing can come
+   * between */
+  const double *norm_in = stage >= 2 ? d->norm_part : NULL;
+  const long norm_count = d->norm_count;
+  d->norm_part = NULL;
+  if (norm_in && d->norm_gen != lg_partials_generation()) lg_fatal("internal: reduction scratch moved inside a merged batch");
 
   /* start of the step: V_eff and the input's reductions */
   if (stage < 2 && (veff || sa->want_energy)) {
@@ -373,12 +382,14 @@ static int tile_step(wf *gwf, const step_args *sa) {
      * `back` times the stored values; the kinetic factors' 1/N accounts for the round trip */
     post = base.back;
   }
+  const double norm_dv = lg_step_factor(g->nx, g->ny, g->nz, g->step) * base.back;
   hgrid_finalize fin;
   memset(&fin, 0, sizeof(fin));
   if (sa->want_energy) {
     hgrid_reduce_job j = {partB, nbB, HGRID_RED_NORM, 3, d->dscal + GS_RED};
     fin.job[fin.njobs++] = j;
   }
+  const int hand_on = (stage == 1 || stage == 2) && sa->want_post_norm && sa->renorm_target > 0.0 && nbB <= 4096;
   long nbpost = nbA;
   for (int half = 0; half < 2; ++half) {
     if ((stage == 1 || stage == 2) && half == 1) break;
@@ -386,6 +397,14 @@ static int tile_step(wf *gwf, const step_args *sa) {
     t = base;
     if (pend) { t.flags |= HGRID_PF_PRESCALE; t.scale = pend; }
     pend = NULL;
+    if (norm_in) {
+      t.flags |= HGRID_PF_PRESCALE;
+      t.norm_partials = norm_in;
+      t.norm_count = norm_count;
+      t.norm_target = sa->renorm_target;
+      t.norm_dv = norm_dv;
+      norm_in = NULL;
+    }
     t.post = post;
     post = 1.0;
     if (sa->tm_im == 0.0) t.flags |= HGRID_PF_KIN_REAL;
@@ -429,7 +448,7 @@ static int tile_step(wf *gwf, const step_args *sa) {
         }
         if ((stage == 1 || stage == 2) && sa->want_post_norm) {
           t.flags |= HGRID_PF_POST_RED;
-          t.partials = partP;
+          t.partials = hand_on ? partH : partP;
           nbpost = nbB;
         }
         lg_run_tile(&t, sa->gpe ? HGRID_TILE_GPE : HGRID_TILE_POT);
@@ -447,22 +466,26 @@ static int tile_step(wf *gwf, const step_args *sa) {
     t.cons = sa->cons;
     lg_run_tile(&t, HGRID_TILE_POT);
   }
-  if (sa->want_post_norm) {
+  if (hand_on) {
+    d->norm_part = partH + HGRID_RED_POST * nbpost;
+    d->norm_count = nbpost;
+    d->norm_gen = lg_partials_generation();
+  } else if (sa->want_post_norm) {
     hgrid_reduce_job j = {partP, nbpost, HGRID_RED_POST, 1, d->dscal + GS_RED + HGRID_RED_POST};
     fin.job[fin.njobs++] = j;
   }
-  if (sa->renorm_target > 0.0) {
+  if (sa->renorm_target > 0.0 && !hand_on) {
     fin.scale = d->dscal + GS_SCALE;
     fin.norm_sum = d->dscal + GS_RED + HGRID_RED_POST;
     fin.target = sa->renorm_target;
-    fin.dv = lg_step_factor(g->nx, g->ny, g->nz, g->step) * base.back;
+    fin.dv = norm_dv;
   } else if (scale) {
     fin.scale = d->dscal + GS_SCALE; /* the pending scale was applied */
   }
   if (fin.njobs || fin.scale) lg_hip(hgrid_step_finalize(&fin), "step_finalize");
   d->valid = GV_DEV;
   d->stamp++;
-  d->pending = sa->renorm_target > 0.0;
+  d->pending = sa->renorm_target > 0.0 && !hand_on;
   d->zpend = defer ? 2 : 0;
   d->kpend = stage == 1 || stage == 2;
   return 1;

@@ -49,6 +49,10 @@ typedef struct grid_dev {
   ktab_cache kin2;         /* the full-step tables of a merged relaxation step (twice that time) */
   int kpend;               /* inside a merged relaxation batch: the array holds the state before
                               the last half kinetic factor of the step (never seen by callers) */
+  const double *norm_part; /* with kpend: the norm's partial sums, from which the next step's first pass
+                              takes its scale (tile passes), in the scratch of generation norm_gen */
+  long norm_count;
+  unsigned long norm_gen;
   ktab_cache kin_energy;   /* |k|^2 tables for energy reductions */
   unsigned long stamp;     /* bumped whenever the device array may have been written */
   void *alt;               /* the data converted to another storage precision (lg_c_in_as) */

@@ -103,3 +103,41 @@ def test_every_2d_geometry(lg, orc, n1):
             print(f"[case] {shape}", flush=True)
             for what, err, bar in steps(lg, orc, shape):
                 assert err < bar, f"{shape} {what}: rel L2 {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", sorted(BARS))
+@pytest.mark.parametrize("shape", [(16, 16, 16), (32, 96, 48), (1, 96, 64), (16, 8, 64), (1, 32, 64)])
+def test_copy_between_steps(lg, shape, prec):
+    """A copy of a state between fused steps, in tile form or a pencil's deferred form and with its
+    normalisation outstanding, holds the values that the grid then shows, and the next step goes on
+    as if there had been no copy: the same kernels on the same values, so to the bit."""
+    rng = np.random.default_rng(sum(shape))
+    psi = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    v = lg.rgrid_alloc(*shape, 0.3, LG.boundary("rgrid_value_outside_periodic"), None, b"v")
+    LG.set_rgrid(v, rng.uniform(0, 1, shape))
+
+    def run(copied):
+        w = lg.grid_wf_alloc(*shape, 0.3, 1.2, LG.WF_PERIODIC_BOUNDARY, LG.WF_2ND_ORDER_FFT, b"w")
+        out = lg.cgrid_alloc(*shape, 0.3, LG.boundary("cgrid_value_outside_periodic"), None, b"out")
+        LG.set_cgrid(w.contents.grid, psi)
+        lg.cgrid_set_precision(w.contents.grid, prec)
+        lg.cgrid_set_precision(out, prec)
+        copies = []
+        for i in range(3):
+            lg.grid_wf_gpe_propagate(w, v, 0.3, LG.c_complex.of(-0.05j), 1)
+            if copied:
+                lg.cgrid_copy(out, w.contents.grid)
+                copies.append(LG.get_cgrid(out))
+        end = LG.get_cgrid(w.contents.grid)
+        lg.cgrid_free(out)
+        lg.grid_wf_free(w)
+        return end, copies
+
+    plain, _ = run(False)
+    end, copies = run(True)
+    lg.rgrid_free(v)
+    assert np.array_equal(end, plain)
+    assert np.array_equal(copies[-1], end)
+    norm = np.sum(np.abs(copies[0]) ** 2) * 0.3 ** sum(n > 1 for n in shape)
+    assert abs(norm - 1.0) < 1e-12 + (1e-6 if prec == b"\x01" else 0.0)
