@@ -1,5 +1,6 @@
 // C-ABI of the pencil FFT passes (see fft_pass.hpp for the kernels).
 #include "fft_pass.hpp"
+#include "row_pass.hpp"
 
 extern "C" int hgrid_fft_supported(long n) {
   if (n >= 2 && n <= 1024 && (n & (n - 1)) == 0) return 1;
@@ -51,6 +52,11 @@ extern "C" int hgrid_fft_pass(const hgrid_pass *p) {
   const bool one = kind == lg::KIND_FFT || kind == lg::KIND_PRE || kind == lg::KIND_FY;
   if (one && p->nfft != 1) return -1;
   if (!one && p->nfft != (skip ? 1 : 2)) return -1;
+  if (kind == lg::KIND_FY && p->axis == 2 && !(p->flags & HGRID_PF_POST_RED) && lg::row::covers(L, p->prec)) {
+    if (p->prec == HGRID_C128) return lg::row::launch_f64(p);
+    if (p->prec == HGRID_C64) return lg::row::launch_f32(p);
+    if (p->prec == HGRID_C64X) return lg::row::launch_f32s_f64(p);
+  }
   if (p->prec == HGRID_C128) return lg::launch_f64(p, L, kind);
   if (p->prec == HGRID_C64) return lg::launch_f32(p, L, kind);
   if (p->prec == HGRID_C64X) return lg::launch_f32s_f64(p, L, kind);
