@@ -158,6 +158,8 @@ typedef struct hgrid_tile {
   int rows, nh;          /* n1 = nh * rows */
   long sx, sh;           /* elements between neighbours along x and h */
   long blocks_a, blocks_b;  /* workgroups of an A-pass and a B-pass (partials per channel) */
+  int threads_a, threads_b; /* of a workgroup */
+  int pencils;           /* bits: pencil passes are faster for 1 steps that end in real space, 2 merged relaxations */
   double back;           /* points along x and h: an inverse after a forward B-pass multiplies by it */
   /* per pass */
   unsigned flags;        /* A: PRESCALE, MID_KRED, KIN_REAL, KCUT, POST_RED

@@ -10,6 +10,7 @@ template <typename C, int LX, int A> static bool plan_b(long points, hgrid_tile 
     using G = GeomB<C, LX, A>;
     if (t->n2 % G::CC) return false;
     t->blocks_b = points / G::T;
+    t->threads_b = G::NT;
     return true;
   } else {
     return false;
@@ -38,10 +39,15 @@ template <typename C> static bool plan_x(long lx, int a, long points, hgrid_tile
 
 // the A-pass tile of rows z rows of lz points: blocks, if its (x, h) groups divide the grid
 template <typename C, int LZ, int B> static bool plan_a(long points, long groups, hgrid_tile *t) {
-  using G = GeomA<C, LZ, B>;
-  if (groups % G::M) return false;
-  t->blocks_a = points / G::T;
-  return true;
+  if constexpr (shape_a<C, LZ, B>()) {
+    using G = GeomA<C, LZ, B>;
+    if (groups % G::M) return false;
+    t->blocks_a = points / G::T;
+    t->threads_a = G::NT;
+    return true;
+  } else {
+    return false;
+  }
 }
 
 template <typename C, int B> static bool plan_z(long points, long groups, hgrid_tile *t) {
@@ -49,8 +55,6 @@ template <typename C, int B> static bool plan_z(long points, long groups, hgrid_
   case n: return plan_a<C, n, B>(points, groups, t);
   switch (t->n2) {
     LG_TILE_LENGTHS(LG_CASE)
-    case 384: if constexpr (B == 4) return t->flat && plan_a<C, 384, 4>(points, groups, t); else return false;
-    case 512: if constexpr (B == 4) return t->flat && plan_a<C, 512, 4>(points, groups, t); else return false;
     default: return false;
   }
 #undef LG_CASE
@@ -69,13 +73,42 @@ template <typename C> static bool plan(hgrid_tile *t) {
   t->back = (double)(t->n0 * t->nh);
   if (!plan_x<C>(t->flat ? t->nh : t->n0, t->flat ? 1 : t->nh, points, t)) return false;
   const long groups = t->n0 * t->nh;
+  bool taken = false;
   switch (t->rows) {
-    case 4: return plan_z<C, 4>(points, groups, t);
-    case 8: return plan_z<C, 8>(points, groups, t);
-    case 16: return plan_z<C, 16>(points, groups, t);
-    case 32: return plan_z<C, 32>(points, groups, t);
-    default: return false;
+    case 4: taken = plan_z<C, 4>(points, groups, t); break;
+    case 8: taken = plan_z<C, 8>(points, groups, t); break;
+    case 16: taken = plan_z<C, 16>(points, groups, t); break;
+    case 32: taken = plan_z<C, 32>(points, groups, t); break;
+    case 64: taken = plan_z<C, 64>(points, groups, t); break;
+    default: break;
   }
+  if (!taken) return false;
+  // Workgroups that fill a CU alone wait for their own loads and stores, which the smaller ones of
+  // the pencil passes overlap; their fewer sweeps gain less then.  ms of 6 steps (relaxation: 32),
+  // pencils and then tiles; GPE in real time, complex potential, the same 4th order, merged
+  // relaxation:
+  //   FP64  256 256 512 (A 1024, B  512 threads) 10.3  9.7   9.3  8.5   12.4 16.3   29.7 30.0
+  //         256 512 256 (   512,   1024)         10.4  8.5   9.5  7.3   12.7 14.9   29.5 25.8
+  //         256 256 256 (   256,   1024)          4.6  3.6   4.1  2.8    5.7  5.5   13.2 10.9
+  //         384 256 384 (   512,    512)         17.2 11.4  14.9  9.7   19.5 15.7   44.8 35.2
+  //   FP32  512 512 512 (  1024,   1024)         26.1 26.5  22.6 18.9   28.6 33.9   77.9 79.9
+  //         512 384 192 (   512,   1024)          7.4  6.9   6.2  4.8    8.0  8.3   21.0 23.4
+  //         256 512 256 (   512,    512)          5.3  5.8   4.3  4.1    5.9  6.9   15.2 15.0
+  //         256 256 512 (   512,    512)          5.5  5.5   4.4  3.8    6.1  6.6   16.5 14.9
+  //         512 256 256 (   256,   1024)          5.5  5.3   4.4  3.3    6.1  6.0   16.0 16.2
+  //         256 256 256 (   256,    512)          2.7  2.1   2.1  1.4    2.8  2.3    7.5  5.9
+  //         384 384 384 (  1024,    768)         11.9 10.4   9.5  8.1   12.1 12.8   36.2 32.5
+  //   FP64  256 192 512 (   512,    512)          7.7  7.4   6.9  6.2    9.2 10.6   22.2 23.2
+  //         512 384 128 (   512,    512)          9.8  7.7   9.0  6.3   11.5 11.1   27.8 24.7
+  //         192 512 256 (  1024,    256)          7.8  6.4   7.2  5.6    9.6 10.4   22.1 21.7
+  const bool f64 = sizeof(C) == 16;
+  const int threads = t->threads_a + t->threads_b;
+  if (!f64 && t->n2 != 384 && t->n1 >= 384 && t->threads_a >= 512 && t->threads_b >= 512) return false;
+  if (threads >= 1024 && (!f64 || t->n0 == 512 || t->n1 == 512 || t->n2 == 512)) t->pencils |= 1;
+  if (f64 && threads >= 1024 && (t->n0 == 512 || t->n2 == 512) && (t->threads_a >= 1024 || (t->nh % 3 == 0 && t->n1 < 384)))
+    t->pencils |= 2;
+  if (!f64 && threads >= 1280 && t->n2 >= 256 && t->n2 != 384) t->pencils |= 2;
+  return true;
 }
 
 }  // namespace tile

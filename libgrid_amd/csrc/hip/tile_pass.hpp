@@ -79,7 +79,9 @@ template <typename C, int LZ, int B> struct GeomA {
                                                      : 8;
   static constexpr int M = T0 / R >= 64 ? 1 : 64 / (T0 / R);
   static constexpr int T = T0 * M, NT = T / R;
-  static constexpr Digits DZ = digits_of(LZ, R), DY = digits_of(B, R);
+  static constexpr Digits DZ = digits_of(LZ, R);
+  // 64 rows 8 x 8: with 16 x 4 the padded exchange of the largest tiles would not fit in LDS
+  static constexpr Digits DY = B == 64 ? Digits{2, {8, 8, 1}} : digits_of(B, R);
   static constexpr int ZLAST = DZ.d[DZ.n - 1];
   static constexpr int PD = ZLAST, PW = 1;  // one spare LDS word per run of the last z digit
   static_assert(DZ.n > 0 && DY.n > 0 && T % R == 0 && NT % 64 == 0, "A-pass geometry");
@@ -376,14 +378,12 @@ template <int NT> __device__ __forceinline__ void reduce_partials(double (&acc)[
 // Waves per SIMD asked of the register allocator: 128 VGPRs for tiles of 16 FP64 or 32 FP32 values
 // per thread (two workgroups of 512 threads per CU).
 template <typename C, int R> constexpr int waves() { return sizeof(C) == 16 ? (R <= 16 ? 4 : 3) : R >= 24 ? 3 : 5; }
-// FP32 data with real factors multiplies in FP64 and needs more
-template <typename C, int R, bool REALK> constexpr int waves_a() { return sizeof(C) == 8 && REALK ? (R >= 24 ? 3 : 4) : waves<C, R>(); }
 
 // ---- A-pass --------------------------------------------------------------------------------------
 
 template <typename C, int LZ, int B, bool REALK>
 __global__ void __launch_bounds__((GeomA<C, LZ, B>::NT))
-__attribute__((amdgpu_waves_per_eu(waves_a<C, GeomA<C, LZ, B>::R, REALK>(), 8))) tile_kinetic(const hgrid_tile a) {
+__attribute__((amdgpu_waves_per_eu(waves<C, GeomA<C, LZ, B>::R>(), 8))) tile_kinetic(const hgrid_tile a) {
   using G = GeomA<C, LZ, B>;
   using Rl = typename real_of<C>::type;
   constexpr int R = G::R, NT = G::NT, M = G::M, T = G::T, PD = G::PD, PW = G::PW;
@@ -470,7 +470,12 @@ __attribute__((amdgpu_waves_per_eu(waves_a<C, GeomA<C, LZ, B>::R, REALK>(), 8)))
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = i0; i < (i0 + 4 < RZ ? i0 + 4 : RZ); ++i) {
-        if constexpr (REALK) v[u * RZ + i] = cscale_d(v[u * RZ + i], t2[kz + ZH * i].x * f.x);
+        if constexpr (REALK) {
+          // hidden from the sum above, with which the compiler would share the values widened to FP64,
+          // all at once (FP32, rows of 512: 145 registers spilled)
+          if constexpr (sizeof(C) == 8) asm volatile("" : "+v"(v[u * RZ + i].x), "+v"(v[u * RZ + i].y));
+          v[u * RZ + i] = cscale_d(v[u * RZ + i], t2[kz + ZH * i].x * f.x);
+        }
         else v[u * RZ + i] = cmul(v[u * RZ + i], round_to<C>(cmul(t2[kz + ZH * i], f)));
       }
     }
@@ -631,10 +636,12 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   auto potential_offset = [&](int t, int u) { return ordered ? (unsigned)(u * SV::r * NT + t) * 8u : real_element(t, u) * 8u; };
   // the start-of-step pass loads vext ahead of the exchange, which hides the latency (256^3 FP64
   // 160 -> 147 us); the potential passes have no registers for it
-  double pv[KIND == TPRE ? R : 1];
+  // 1024 threads of 32 values have no registers for the potential of all of them
+  constexpr bool FULL = NT == 1024 && R == 32;
+  double pv[KIND == TPRE && !FULL ? R : 1];
   auto load_potential = [&]() {
-    if constexpr (KIND == TPRE) {
-  #pragma unroll
+    if constexpr (KIND == TPRE && !FULL) {
+#pragma unroll
       for (int u = 0; u < R / SV::r; ++u) {
         const unsigned e = potential_offset(tid, u);
 #pragma unroll
@@ -668,14 +675,16 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   if constexpr (KIND == TPRE) {
 #pragma unroll
     for (int u = 0; u < R / SV::r; ++u) {
+      const unsigned e = FULL ? potential_offset(tid, u) : 0;
+      if constexpr (FULL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < SV::r; ++i) {
-        const double d = cnorm2(v[u * SV::r + i]);
-        if (fl & HGRID_PF_PRE_VEFF) bstore_f64(pv[u * SV::r + i] + a.g * d, rveff, (unsigned)tid * 8u, (unsigned)((u * SV::r + i) * NT) * 8u);
+        const double d = cnorm2(v[u * SV::r + i]), pe = FULL ? bload_f64(rpv, e, (unsigned)i * steppv) : pv[FULL ? 0 : u * SV::r + i];
+        if (fl & HGRID_PF_PRE_VEFF) bstore_f64(pe + a.g * d, rveff, (unsigned)tid * 8u, (unsigned)((u * SV::r + i) * NT) * 8u);
         if (fl & HGRID_PF_PRE_RED) {
           acc[HGRID_RED_NORM] += d;
           acc[HGRID_RED_QUART] += d * d;
-          acc[HGRID_RED_VEXT] += pv[u * SV::r + i] * d;
+          acc[HGRID_RED_VEXT] += pe * d;
         }
       }
     }
@@ -714,11 +723,15 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
       for (int u = 0; u < R / SV::r; ++u) {
         const unsigned e = potential_offset(tid, u);
         double p[SV::r];
+        auto fetch = [&](int i0, int n) {
 #pragma unroll
-        for (int i = 0; i < SV::r; ++i) p[i] = a.cons + bload_f64(rpv, e, (unsigned)i * steppv);
+          for (int i = i0; i < i0 + n; ++i) p[i] = a.cons + bload_f64(rpv, e, (unsigned)i * steppv);
+        };
+        if constexpr (!FULL) fetch(0, SV::r);
 #pragma unroll
         for (int i0 = 0; i0 < SV::r; i0 += GROUP) {
           __builtin_amdgcn_sched_barrier(0);
+          if constexpr (FULL) fetch(i0, GROUP);
 #pragma unroll
           for (int i = i0; i < (i0 + GROUP < SV::r ? i0 + GROUP : SV::r); ++i) apply(v[u * SV::r + i], p[i]);
         }
@@ -764,20 +777,31 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
 // overlap each other's loads, exchanges and stores: 256^3 A-pass 107 us, against 147 with 32 rows
 // (512 threads); the B-pass then has 16 h and 1024 threads, 211 against 190 us, and the whole
 // Gross-Pitaevskii step 580 against 611.  In FP32 32 rows from 192 on (256^3 step 378 against 400).
+// The longer axes take what fits: a tile of at most 2^15 FP32 or 2^14 FP64 values (768 threads of 24),
+// with 64-byte rows in the B-pass.
 constexpr int rows_of(bool f64, long n0, long n1) {
   return n1 == 16                                        ? 4
          : n1 == 24 || n1 == 32                          ? 8
          : n1 == 48 || n1 == 64 || n1 == 96 || n1 == 128 ? 16
-         : n1 == 192                                     ? (f64 ? 16 : 32)
-         : n1 == 256                                     ? (f64 && n0 % 3 != 0 ? 16 : 32)
+         : n1 == 192                                     ? (f64 && n0 <= 256 ? 16 : 32)
+         : n1 == 256                                     ? (f64 && n0 <= 256 && n0 % 3 != 0 ? 16 : 32)
+         : n1 == 384                                     ? (f64 && n0 <= 256 ? 32 : 64)
+         : n1 == 512                                     ? (f64 && n0 <= 256 && n0 % 3 != 0 ? 32 : 64)
                                                          : 0;
 }
-// the (x, h) shapes that a B-pass is built for
-template <typename C, int LX, int A> constexpr bool shape_b() {
-  return A == 16 ? sizeof(C) == 16 && LX % 3 != 0 : A == 12 ? sizeof(C) == 16 : true;
+// the tiles that passes are built for
+template <typename G, typename C> constexpr bool fits() {
+  return G::NT <= (sizeof(C) == 16 && G::R == 24 ? 768 : 1024);
 }
+template <typename C, int LX, int A> constexpr bool shape_b() {
+  if constexpr (A == 16 ? sizeof(C) == 8 || LX % 3 == 0 || LX > 256 : A == 12 ? sizeof(C) == 8 || LX > 256 : A == 1 ? LX > 256 : false)
+    return false;
+  else
+    return fits<GeomB<C, LX, A>, C>();
+}
+template <typename C, int LZ, int B> constexpr bool shape_a() { return fits<GeomA<C, LZ, B>, C>(); }
 
-#define LG_TILE_LENGTHS(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
+#define LG_TILE_LENGTHS(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 
 int launch_kinetic_f64(const hgrid_tile *p);
 int launch_kinetic_f32(const hgrid_tile *p);
@@ -791,13 +815,17 @@ int launch_gpr_f64(const hgrid_tile *p);
 int launch_gpr_f32(const hgrid_tile *p);
 
 template <typename C, int LZ, int B> int launch_a(const hgrid_tile *p) {
-  using G = GeomA<C, LZ, B>;
-  const long nb = p->n0 * p->n1 * p->n2 / G::T;
-  if (p->flags & HGRID_PF_KIN_REAL)
-    hipLaunchKernelGGL((tile_kinetic<C, LZ, B, true>), dim3((unsigned)nb), dim3(G::NT), 0, stream(), *p);
-  else
-    hipLaunchKernelGGL((tile_kinetic<C, LZ, B, false>), dim3((unsigned)nb), dim3(G::NT), 0, stream(), *p);
-  return check_launch("tile_kinetic");
+  if constexpr (shape_a<C, LZ, B>()) {
+    using G = GeomA<C, LZ, B>;
+    const long nb = p->n0 * p->n1 * p->n2 / G::T;
+    if (p->flags & HGRID_PF_KIN_REAL)
+      hipLaunchKernelGGL((tile_kinetic<C, LZ, B, true>), dim3((unsigned)nb), dim3(G::NT), 0, stream(), *p);
+    else
+      hipLaunchKernelGGL((tile_kinetic<C, LZ, B, false>), dim3((unsigned)nb), dim3(G::NT), 0, stream(), *p);
+    return check_launch("tile_kinetic");
+  } else {
+    return -1;
+  }
 }
 
 template <typename C, int B> int launch_a_rows(const hgrid_tile *p) {
@@ -805,14 +833,9 @@ template <typename C, int B> int launch_a_rows(const hgrid_tile *p) {
   case n: return launch_a<C, n, B>(p);
   switch (p->n2) {
     LG_TILE_LENGTHS(LG_CASE)
-    default: break;
+    default: return -1;
   }
 #undef LG_CASE
-  if constexpr (B == 4) {  // 2-D grids
-    if (p->n2 == 384) return launch_a<C, 384, 4>(p);
-    if (p->n2 == 512) return launch_a<C, 512, 4>(p);
-  }
-  return -1;
 }
 
 template <typename C> int launch_kinetic(const hgrid_tile *p) {
@@ -821,6 +844,7 @@ template <typename C> int launch_kinetic(const hgrid_tile *p) {
     case 8: return launch_a_rows<C, 8>(p);
     case 16: return launch_a_rows<C, 16>(p);
     case 32: return launch_a_rows<C, 32>(p);
+    case 64: return launch_a_rows<C, 64>(p);
     default: return -1;
   }
 }

@@ -327,8 +327,9 @@ static int tile_step(wf *gwf, const step_args *sa) {
   /* complex time with a real potential stays with the pencils */
   if ((sa->gpe && sa->c_re != 0.0 && sa->c_im != 0.0) || !lg_tile_init(&base, &s, d->prec, NULL)) return 0;
   const double *scale;
-  base.psi = lg_c_raw(g, &scale);
   const int defer = !sa->no_defer, stage = sa->stage;
+  if ((!defer && (base.pencils & 1)) || (stage && (base.pencils & 2))) return 0;
+  base.psi = lg_c_raw(g, &scale);
   if (stage && (!defer || sa->gpe != 1 || sa->g != 0.0 || (stage >= 2 && (d->zpend != 2 || !d->kpend || sa->want_energy))))
     lg_fatal("internal: merged relaxation stage %d on a state it does not apply to", stage);
   if (stage <= 1 && d->kpend) lg_fatal("internal: a merged relaxation batch was left unfinished");

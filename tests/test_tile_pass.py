@@ -30,8 +30,12 @@ def test_shapes_taken_and_left():
             assert planned(prec, n, n, n), (prec, n)
         assert not planned(LG.HGRID_C64X, n, n, n)  # FP32 storage with FP64 arithmetic
     assert planned(LG.HGRID_C128, 1, 384, 512) and planned(LG.HGRID_C64, 1, 1024, 64)
-    for shape in ((8, 64, 64), (64, 12, 64), (64, 64, 512), (512, 64, 64), (64, 512, 64), (1, 1, 64), (1, 32, 64),
-                  (64, 384, 64), (1, 64, 24)):
+    for shape in ((64, 64, 512), (512, 64, 64), (64, 512, 64), (384, 256, 512)):
+        assert planned(LG.HGRID_C128, *shape) and planned(LG.HGRID_C64, *shape), shape
+    # one tile would be 2^15 FP64 values, twice what a CU's registers hold; in FP32 pencils are faster
+    assert not planned(LG.HGRID_C128, 512, 512, 512) and not planned(LG.HGRID_C64, 512, 512, 512)
+    assert planned(LG.HGRID_C64, 64, 512, 512) and planned(LG.HGRID_C64, 384, 384, 384)
+    for shape in ((8, 64, 64), (64, 12, 64), (1, 1, 64), (1, 32, 64), (64, 1024, 64), (64, 64, 1024), (1, 64, 24)):
         assert not planned(LG.HGRID_C128, *shape), shape
 
 
@@ -91,6 +95,19 @@ def test_every_tile_geometry(lg, orc, axis, n1):
         print(f"[case] {shape}", flush=True)
         for what, err, bar in steps(lg, orc, shape):
             assert err < bar, f"{shape} {what}: rel L2 {err:.3e}"
+
+
+LONG = [(n, n1, 16) for n in (384, 512) for n1 in (16, 48, 96, 128, 192, 256, 384, 512)]
+LONG += [(16, n1, n) for n in (384, 512) for n1 in (16, 32, 64, 256, 384, 512)]
+LONG += [(n, n1, 32) for n in (16, 256) for n1 in (384, 512)] + [(16, 512, n) for n in LENGTHS] + [(24, 512, 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", LONG)
+def test_long_axes(lg, orc, shape):
+    """Axes of 384 and 512 points: the same, and every z with the 64 rows of the longest middle axes."""
+    for what, err, bar in steps(lg, orc, shape):
+        assert err < bar, f"{shape} {what}: rel L2 {err:.3e}"
 
 
 @pytest.mark.gpu
