@@ -150,7 +150,7 @@ int hgrid_fft_supported(long n);
  * A 2-D grid has no x: its h takes x's place (flat). */
 typedef struct hgrid_tile {
   void *psi;             /* device array (complex, precision prec), transformed in place */
-  void *out;             /* HGRID_TILE_POT: another array for the result (NULL: in place) */
+  void *out;             /* KINETIC, POT, MERGE: another array for the result (NULL: in place) */
   int prec;              /* HGRID_C128 / HGRID_C64 */
   long n0, n1, n2;       /* squeezed shape; n2 is contiguous */
   /* filled in by hgrid_tile_plan */
@@ -182,12 +182,16 @@ typedef struct hgrid_tile {
   double *veff;          /* V_eff in the order of the B-pass's threads (n0 n1 n2 doubles) */
   double g, c_re, c_im, cons;
   double *partials;
+  const void *merge;     /* MERGE: a state in real space, which may be out */
+  long bounds[6];        /* MERGE: lx hx ly hy lz hz of the absorbing boundary */
 } hgrid_tile;
 
 enum { HGRID_TILE_KINETIC = 0,   /* A-pass */
        HGRID_TILE_START = 1,     /* B-pass: inverse, V_eff / reductions, nothing else stored */
        HGRID_TILE_POT = 2,       /* B-pass with a complex potential or none */
-       HGRID_TILE_GPE = 3 };     /* B-pass with V_eff, or vext where veff is NULL; c real or imaginary */
+       HGRID_TILE_GPE = 3,       /* B-pass with V_eff, or vext where veff is NULL; c real or imaginary */
+       HGRID_TILE_MERGE = 4 };   /* B-pass of a 3-D grid: between its transforms psi becomes
+                                  * ((1 - alpha) merge + alpha psi) / back, alpha the absorbing amplitude */
 
 /* Whether tile passes cover this shape and precision; fills in the geometry. */
 int hgrid_tile_plan(int prec, long n0, long n1, long n2, hgrid_tile *t);

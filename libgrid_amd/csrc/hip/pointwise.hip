@@ -11,6 +11,7 @@
 // grid_wf_density (src/grid_wf.c:611-627), grid_real_to_complex_re (src/ngrid.c:53-80),
 // cgrid_fd_laplace (src/cgrid_diff.c:303-330) with the boundary rules of src/cgrid_bc.c:21-86.
 
+#include "absorb.hpp"
 #include "cx.hpp"
 #include "grid_hip.h"
 #include "phase_math.hpp"
@@ -290,20 +291,6 @@ __global__ void k_kinetic_phase(C *psi, long nx, long ny, long nz, const double2
   }
 }
 
-// absorbing-boundary amplitude: 0 inside [lx, hx] x [ly, hy] x [lz, hz]; outside, the distance
-// over the lower bound per axis (both sides), summed, times 2/3, capped at 1
-__device__ static double absorb_amp(long i, long j, long k, long lx, long hx, long ly, long hy, long lz, long hz) {
-  double t = 0.0;
-  if (i < lx) t += (double)(lx - i) / (double)lx;
-  else if (i > hx) t += (double)(i - hx) / (double)lx;
-  if (j < ly) t += (double)(ly - j) / (double)ly;
-  else if (j > hy) t += (double)(j - hy) / (double)ly;
-  if (k < lz) t += (double)(lz - k) / (double)lz;
-  else if (k > hz) t += (double)(k - hz) / (double)lz;
-  t *= 2.0 / 3.0;
-  return t > 1.0 ? 1.0 : t;
-}
-
 // dst = (1 - alpha) wr + alpha wi (dst may be wr); products and sums rounded separately
 template <typename C>
 __global__ void k_wf_merge(C *dst, const C *wr, const C *wi, long nx, long ny, long nz, long lx, long hx, long ly,
@@ -312,7 +299,7 @@ __global__ void k_wf_merge(C *dst, const C *wr, const C *wi, long nx, long ny, l
   const long n = nx * ny * nz;
   LG_GRID_STRIDE(idx, n) {
     const long i = idx / (ny * nz), j = (idx / nz) % ny, k = idx % nz;
-    const double al = absorb_amp(i, j, k, lx, hx, ly, hy, lz, hz), bl = 1.0 - al;
+    const double al = absorb_sum(absorb_part(i, lx, hx), absorb_part(j, ly, hy), absorb_part(k, lz, hz)), bl = 1.0 - al;
     const C r = wr[idx], m = wi[idx];
     const double re = bl * (double)r.x + al * (double)m.x, im = bl * (double)r.y + al * (double)m.y;
     dst[idx] = mk<C>((typename real_of<C>::type)re, (typename real_of<C>::type)im);

@@ -137,6 +137,9 @@ extern "C" int hgrid_tile_pass(const hgrid_tile *t, int pass) {
     case HGRID_TILE_KINETIC: return f64 ? lg::tile::launch_kinetic_f64(t) : lg::tile::launch_kinetic_f32(t);
     case HGRID_TILE_START: return f64 ? lg::tile::launch_pre_f64(t) : lg::tile::launch_pre_f32(t);
     case HGRID_TILE_POT: return f64 ? lg::tile::launch_pot_f64(t) : lg::tile::launch_pot_f32(t);
+    case HGRID_TILE_MERGE:
+      if (!t->merge || t->flat) return -1;
+      return f64 ? lg::tile::launch_mrg_f64(t) : lg::tile::launch_mrg_f32(t);
     case HGRID_TILE_GPE:
       if ((!t->veff && !t->vext) || (t->c_re != 0.0 && t->c_im != 0.0)) return -1;
       if (t->c_im == 0.0) return f64 ? lg::tile::launch_gpr_f64(t) : lg::tile::launch_gpr_f32(t);

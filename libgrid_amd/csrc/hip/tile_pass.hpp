@@ -25,6 +25,7 @@
 // transform is ever put into natural order.  Each wave holds whole pencils of an axis, so the
 // exchanges between its digits are the wave's own; only those between axes need the workgroup.
 #pragma once
+#include "absorb.hpp"
 #include "fft_pass.hpp"
 
 namespace lg {
@@ -498,11 +499,12 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomA<C, LZ, B>::R>(), 8))) tile_kin
 #pragma unroll
     for (int j = 0; j < R; ++j) acc[HGRID_RED_POST] += cnorm2(v[j]);
   }
+  const auto rout = make_rsrc((const C *)(a.out ? a.out : a.psi) + (long)blockIdx.x * T, (unsigned long)T * CS);
 #pragma unroll
   for (int u = 0; u < R / Y0::r; ++u) {
     const unsigned b = (unsigned)Y0::lin(tid, u) * CS;
 #pragma unroll
-    for (int i = 0; i < Y0::r; ++i) bstore<C>(v[u * Y0::r + i], rio, b, (unsigned)(i * Y0::s) * CS);
+    for (int i = 0; i < Y0::r; ++i) bstore<C>(v[u * Y0::r + i], rout, b, (unsigned)(i * Y0::s) * CS);
   }
   if (fl & (HGRID_PF_MID_KRED | HGRID_PF_POST_RED)) reduce_partials<NT>(acc, tid, a.partials);
 }
@@ -515,7 +517,9 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomA<C, LZ, B>::R>(), 8))) tile_kin
 // TGPE / TGPR: the same with a real potential, real time (imaginary c) / imaginary time (real c).  A
 //       kernel with the general complex c beside them spilled 48 of 128 VGPRs (256^3 FP64 real-time
 //       pass 309 us); complex time with a real potential stays with the pencil passes
-enum { TPRE = 0, TPOT = 1, TGPE = 2, TGPR = 3 };
+//   TMRG inverse, merge with another real-space state by the absorbing boundary's amplitude, forward:
+//       in place of an inverse pass, a merge over three arrays and the next step's forward pass
+enum { TPRE = 0, TPOT = 1, TGPE = 2, TGPR = 3, TMRG = 4 };
 
 template <typename C, int LX, int A, int KIND>
 __global__ void __launch_bounds__((GeomB<C, LX, A>::NT))
@@ -579,7 +583,7 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   };
   auto store = [&](auto stage, unsigned step, auto &&at) {
     using S = decltype(stage);
-    const auto rout = make_rsrc(KIND == TPOT && a.out ? a.out : a.psi, ntot * CS);
+    const auto rout = make_rsrc((KIND == TPOT || KIND == TMRG) && a.out ? a.out : a.psi, ntot * CS);
 #pragma unroll
     for (int u = 0; u < R / S::r; ++u) {
       const unsigned e = at(tid, u);
@@ -690,17 +694,17 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
     }
     if (fl & HGRID_PF_PRE_RED) reduce_partials<NT>(acc, tid, a.partials);
     return;
-  } else if constexpr (KIND == TPOT) {
-    if (a.pot) {
-      // four values ahead of the factors that use them
-      const auto rpot = make_rsrc(a.pot, ntot * CS);
+  } else if constexpr (KIND == TPOT || KIND == TMRG) {
+    // values of another array at the tile's real-space elements, four ahead of their use
+    auto with_values = [&](const void *array, auto &&apply) {
+      const auto ro = make_rsrc(array, ntot * CS);
       constexpr int AHEAD = R % 4 == 0 ? 4 : R;
       C p[2][AHEAD];
       auto fetch = [&](int j0, C(&q)[AHEAD]) {
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
           const int u = (j0 + j) / SV::r, i = (j0 + j) % SV::r;
-          q[j] = bload<C>(rpot, real_element(tid, u) * CS, (unsigned)i * stepv * CS);
+          q[j] = bload<C>(ro, real_element(tid, u) * CS, (unsigned)i * stepv * CS);
         }
       };
       fetch(0, p[0]);
@@ -711,11 +715,35 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
           if (j % GROUP == 0) __builtin_amdgcn_sched_barrier(0);
-          const C q = p[(j0 / AHEAD) % 2][j];
-          v[j0 + j] = cmul(v[j0 + j], phase_factor<C>(a.c_re, a.c_im, a.cons + (double)q.x, (double)q.y));
+          v[j0 + j] = apply(v[j0 + j], p[(j0 / AHEAD) % 2][j], (j0 + j) / SV::r, (j0 + j) % SV::r);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (KIND == TPOT) {
+      if (a.pot) {
+        with_values(a.pot, [&](C c, C q, int, int) {
+          return cmul(c, phase_factor<C>(a.c_re, a.c_im, a.cons + (double)q.x, (double)q.y));
+        });
+      }
+    } else {
+      // the amplitude's shares of x, h and z, from LDS: formed in every thread their divisions spilled
+      // up to 265 registers.  The other state's values arrive before the exchange's barrier, behind
+      // which the tile's own elements of it, where out is that array, are overwritten.
+      static_assert(sizeof(lds) >= (LX + A + CC) * sizeof(double) || A == 1, "room for the shares");
+      volatile double *share = (volatile double *)lds;
+      tile_sync<NT>();
+      for (int e = tid; e < LX + A + CC; e += NT)
+        share[e] = e < LX       ? absorb_part(e, a.bounds[0], a.bounds[1])
+                   : e < LX + A ? absorb_part((long)l + (long)(e - LX) * a.rows, a.bounds[2], a.bounds[3])
+                                : absorb_part((long)z0 + (e - LX - A), a.bounds[4], a.bounds[5]);
+      tile_sync<NT>();
+      with_values(a.merge, [&](C m, C r, int u, int i) {
+#pragma clang fp contract(off)
+        const int lin = SV::lin(tid, u);
+        const double al = absorb_sum(share[lin / (A * CC)], share[LX + i], share[LX + A + lin % CC]), bl = 1.0 - al;
+        return mk<C>((Rl)((bl * (double)r.x + al * (double)m.x) * a.post), (Rl)((bl * (double)r.y + al * (double)m.y) * a.post));
+      });
     }
   } else {
     auto factors = [&](auto &&apply) {
@@ -809,6 +837,8 @@ int launch_pre_f64(const hgrid_tile *p);
 int launch_pre_f32(const hgrid_tile *p);
 int launch_pot_f64(const hgrid_tile *p);
 int launch_pot_f32(const hgrid_tile *p);
+int launch_mrg_f64(const hgrid_tile *p);
+int launch_mrg_f32(const hgrid_tile *p);
 int launch_gpe_f64(const hgrid_tile *p);
 int launch_gpe_f32(const hgrid_tile *p);
 int launch_gpr_f64(const hgrid_tile *p);
@@ -850,7 +880,7 @@ template <typename C> int launch_kinetic(const hgrid_tile *p) {
 }
 
 template <typename C, int LX, int A, int KIND> int launch_b(const hgrid_tile *p) {
-  if constexpr (shape_b<C, LX, A>()) {
+  if constexpr (shape_b<C, LX, A>() && (KIND != TMRG || A > 1)) {
     using G = GeomB<C, LX, A>;
     const long nb = p->n0 * p->n1 * p->n2 / G::T;
     hipLaunchKernelGGL((tile_potential<C, LX, A, KIND>), dim3((unsigned)nb), dim3(G::NT), 0, stream(), *p);

@@ -751,6 +751,95 @@ static void check_fft_grid(cgrid *g) {
 }
 
 static void propagate_split(wf *gwf, cgrid *potential, REAL complex time, int real_space);
+static void split_args(wf *gwf, cgrid *potential, REAL complex time, step_args *sa);
+
+/* A step with an absorbing boundary in tile passes: psi's real-time step (args[0]) and the
+ * imaginary-time step (args[1]) of the same state into w share the forward transform, and the last
+ * B-pass merges the two and leaves the result in tile form.  Four A- and four B-passes a step
+ * replace a copy, twice five passes from and to real space and a merge: 96 x 192 x 128 in FP64
+ * 190 us a step against 233 (and 340 in pencil passes); faster in every shape of tile passes that
+ * was timed, also where those ending in real space are slower than pencils (256 x 256 x 512 FP64 by
+ * 1.07, 256^3 by 1.39, 64^3 by 2.06). */
+static int tile_absorb_step(wf *gwf, cgrid *w, const step_args *args) {
+  cgrid *g = gwf->grid;
+  grid_dev *d = g->dev;
+  lg_shape s;
+  lg_squeeze(g->nx, g->ny, g->nz, &s);
+  hgrid_tile base, t;
+  if (s.m != 3 || !args[0].pot || !lg_tile_init(&base, &s, d->prec, NULL)) return 0;
+  if (d->zpend == 1) lg_c_materialize(g);
+  const double *scale;
+  void *psi = lg_c_raw(g, &scale);
+  const double *pend = scale;
+  void *other = lg_c_out(w);
+  w->step = g->step;
+  w->x0 = g->x0;
+  w->y0 = g->y0;
+  w->z0 = g->z0;
+  w->kx0 = g->kx0;
+  w->ky0 = g->ky0;
+  w->kz0 = g->kz0;
+  double post = base.back;
+  if (!d->zpend) {
+    t = base;
+    t.psi = psi;
+    t.flags = HGRID_PF_POT_NOFFT1 | (pend ? HGRID_PF_PRESCALE : 0);
+    t.scale = pend;
+    lg_run_tile(&t, HGRID_TILE_POT);
+    pend = NULL;
+    post = 1.0;
+  }
+  for (int which = 1; which >= 0; --which) { /* the copy first: its first pass reads psi */
+    const step_args *sa = &args[which];
+    cgrid *to = which ? w : g;
+    ktab_cache *kt = lg_kinetic_tables(to, sa->tm_re, sa->tm_im, g->fft_norm);
+    for (int half = 0; half < 2; ++half) {
+      t = base;
+      t.psi = which && half ? other : psi;
+      t.out = which ? other : psi;
+      if (!half) {
+        t.flags = pend ? HGRID_PF_PRESCALE : 0;
+        t.scale = pend;
+        t.post = post;
+      }
+      if (sa->tm_im == 0.0) t.flags |= HGRID_PF_KIN_REAL;
+      t.ktab_0 = sq(kt->t, &s, g, 0);
+      t.ktab_1 = sq(kt->t, &s, g, 1);
+      t.ktab_2 = sq(kt->t, &s, g, 2);
+      if (sa->kcut) {
+        t.flags |= HGRID_PF_KCUT;
+        t.kc_0 = sq((void *const *)kt->kc, &s, g, 0);
+        t.kc_1 = sq((void *const *)kt->kc, &s, g, 1);
+        t.kc_2 = sq((void *const *)kt->kc, &s, g, 2);
+        t.kcut2 = sa->kcut2;
+      }
+      lg_run_tile(&t, HGRID_TILE_KINETIC);
+      if (half) continue;
+      t = base;
+      t.psi = which ? other : psi;
+      t.pot = sa->pot;
+      t.c_re = sa->c_re;
+      t.c_im = sa->c_im;
+      t.cons = sa->cons;
+      lg_run_tile(&t, HGRID_TILE_POT);
+    }
+  }
+  t = base;
+  t.psi = psi;
+  t.flags = HGRID_PF_POT_NOFFT2;
+  lg_run_tile(&t, HGRID_TILE_POT);
+  t = base;
+  t.psi = other;
+  t.merge = t.out = psi;
+  t.post = 1.0 / base.back;
+  const long bounds[6] = {gwf->lx, gwf->hx, gwf->ly, gwf->hy, gwf->lz, gwf->hz};
+  memcpy(t.bounds, bounds, sizeof(bounds));
+  lg_run_tile(&t, HGRID_TILE_MERGE);
+  lg_c_written(g, 1);
+  d->zpend = 2;
+  lg_c_written(w, 1);
+  return 1;
+}
 
 void grid_wf_propagate(wf *gwf, cgrid *potential, REAL complex time) {
   cgrid *g = gwf->grid;
@@ -765,6 +854,13 @@ void grid_wf_propagate(wf *gwf, cgrid *potential, REAL complex time) {
       gwf->cworkspace = cgrid_alloc(g->nx, g->ny, g->nz, g->step, g->value_outside, g->outside_params_ptr, "WF cworkspace 1");
     cgrid *w = gwf->cworkspace;
     if (cgrid_get_precision(w) != cgrid_get_precision(g)) cgrid_set_precision(w, cgrid_get_precision(g));
+    if (lg_cdev(g) && w != potential && g != potential) {
+      check_fft_grid(g);
+      step_args args[2];
+      split_args(gwf, potential, time, &args[0]);
+      split_args(gwf, potential, -I * creal(time), &args[1]);
+      if (tile_absorb_step(gwf, w, args)) return;
+    }
     cgrid_copy(w, g);
     REAL (*save)(INT, INT, INT, INT, INT, INT, INT, INT, INT) = gwf->ts_func;
     gwf->ts_func = NULL;
@@ -779,27 +875,18 @@ void grid_wf_propagate(wf *gwf, cgrid *potential, REAL complex time) {
   propagate_split(gwf, potential, time, 0);
 }
 
-/* one split-operator step of gwf->grid by the propagator's sequence; real_space leaves the
- * result untransformed (the absorbing-boundary merge reads it) */
-static void propagate_split(wf *gwf, cgrid *potential, REAL complex time, int real_space) {
+/* the arguments of a split-operator step of gwf->grid by the propagator's sequence */
+static void split_args(wf *gwf, cgrid *potential, REAL complex time, step_args *sa) {
   cgrid *g = gwf->grid;
   const REAL kx0 = g->kx0, ky0 = g->ky0, kz0 = g->kz0;
   const REAL cons = -(HBAR * HBAR / (2.0 * gwf->mass)) * (kx0 * kx0 + ky0 * ky0 + kz0 * kz0);
-  check_fft_grid(g);
-  lg_shape s;
-  lg_squeeze(g->nx, g->ny, g->nz, &s);
-  if (s.m < 2) {
-    split_step_unfused(gwf, potential, time, cons);
-    return;
-  }
-  step_args sa;
-  memset(&sa, 0, sizeof(sa));
+  memset(sa, 0, sizeof(*sa));
   if (potential) {
     if (potential->nx != g->nx || potential->ny != g->ny || potential->nz != g->nz)
       lg_fatal("grid_wf_propagate: potential and wavefunction grids differ in size");
     /* the potential keeps its own precision (a copy in the state's storage precision is used),
      * so an FP64 state propagated with it later still sees the FP64 values */
-    sa.pot = lg_c_in_as(potential, g->dev->prec);
+    sa->pot = lg_c_in_as(potential, g->dev->prec);
   }
   /* 4th order (reference src/grid_wf.c:433-457): the outer V(t/6) stages ride on the first
    * and last z passes of a fused K(t/2) V(2t/3) K(t/2).  The reference also forms
@@ -807,21 +894,37 @@ static void propagate_split(wf *gwf, cgrid *potential, REAL complex time, int re
    * potential to the V(2t/3) stage (:452); that term never reaches psi, so it is not formed. */
   const int fourth = fourth_order(gwf);
   const REAL complex tv = fourth ? 2.0 * time / 3.0 : time;
-  if (fourth && sa.pot) {
+  if (fourth && sa->pot) {
     const REAL complex t6 = time / 6.0;
-    sa.pot6 = sa.pot;
-    sa.c6_re = cimag(t6) / HBAR;
-    sa.c6_im = -creal(t6) / HBAR;
+    sa->pot6 = sa->pot;
+    sa->c6_re = cimag(t6) / HBAR;
+    sa->c6_im = -creal(t6) / HBAR;
   }
-  sa.c_re = cimag(tv) / HBAR;
-  sa.c_im = -creal(tv) / HBAR;
-  sa.cons = cons;
+  sa->c_re = cimag(tv) / HBAR;
+  sa->c_im = -creal(tv) / HBAR;
+  sa->cons = cons;
   const REAL complex tm = -I * (0.5 * time) * HBAR / (gwf->mass * 2.0);
-  sa.tm_re = creal(tm);
-  sa.tm_im = cimag(tm);
-  sa.kcut = uses_cutoff(gwf);
-  sa.kcut2 = gwf->kmax * gwf->kmax;
-  sa.no_defer = fourth || real_space; /* the last V(t/6) stage and the merge act in real space */
+  sa->tm_re = creal(tm);
+  sa->tm_im = cimag(tm);
+  sa->kcut = uses_cutoff(gwf);
+  sa->kcut2 = gwf->kmax * gwf->kmax;
+}
+
+/* one split-operator step of gwf->grid by the propagator's sequence; real_space leaves the
+ * result untransformed (the absorbing-boundary merge reads it) */
+static void propagate_split(wf *gwf, cgrid *potential, REAL complex time, int real_space) {
+  cgrid *g = gwf->grid;
+  check_fft_grid(g);
+  lg_shape s;
+  lg_squeeze(g->nx, g->ny, g->nz, &s);
+  if (s.m < 2) {
+    const REAL kx0 = g->kx0, ky0 = g->ky0, kz0 = g->kz0;
+    split_step_unfused(gwf, potential, time, -(HBAR * HBAR / (2.0 * gwf->mass)) * (kx0 * kx0 + ky0 * ky0 + kz0 * kz0));
+    return;
+  }
+  step_args sa;
+  split_args(gwf, potential, time, &sa);
+  sa.no_defer = fourth_order(gwf) || real_space; /* the last V(t/6) stage and the merge act in real space */
   fused_step(gwf, &sa);
 }
 

@@ -81,6 +81,18 @@ def steps(lg, orc, shape):
         for prec, bar in BARS.items():
             got = run(prec, prop, lambda w: lg.grid_wf_propagate(w, vp, LG.c_complex.of(0.02)))
             yield f"propagate {name} precision {prec[0]}", rel_l2(got, ref), bar
+    if min(shape) > 1:  # absorbing boundary: two such steps of either time a step, and their merge
+        bounds = [b for n in shape for b in (n // 4, n - 1 - n // 4)]
+        ref = psi.copy()
+        for _ in range(2):
+            orc.wf_propagate_absorb_inplace(ref, pot, step, mass, k0, 0.02, tuple(bounds), None)
+
+        def absorbed(w):
+            lg.grid_wf_boundary(w, None, *bounds)
+            lg.grid_wf_propagate(w, vp, LG.c_complex.of(0.02))
+
+        for prec, bar in BARS.items():
+            yield f"absorbing precision {prec[0]}", rel_l2(run(prec, LG.WF_2ND_ORDER_FFT, absorbed), ref), 2 * bar
     lg.cgrid_free(vp)
     lg.rgrid_free(vr)
 
