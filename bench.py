@@ -6,7 +6,7 @@ complex128 grid, spacing 0.25 bohr: V_eff = 0.5*0.01*r^2 + 0.05*exp(-r^2/4) + 0.
 built from the start-of-step state, K(dt/2) V(dt) K(dt/2) with dt = 0.05, renormalisation,
 and the energy of the start-of-step state — libgrid's grid_wf_gpe_propagate, i.e. the
 reference composition grid_wf_density -> grid_real_to_complex_re -> grid_wf_propagate ->
-grid_wf_normalize fused into 9 pencil passes.  Inputs are synthetic (seeded) and resident in
+grid_wf_normalize fused into 4 passes.  Inputs are synthetic (seeded) and resident in
 HBM before timing starts.
 
 Prints one JSON line with steps/s, the roofline of the dominant kernel (HIP events on the
@@ -33,8 +33,13 @@ def log(msg):
 
 
 def classify_pass(LG, axis, nfft, flags):
-    """Name of a pass kind of the fused GPE step from its axis (0 outer, 2 contiguous), number of
-    transforms and flags."""
+    """Name of a pass kind of the fused GPE step from its axis (0 outer, 2 contiguous; 3 and 4 the
+    tile passes over rows and z, and over x and h), number of transforms and flags."""
+    if axis == 3:
+        return "tile_kin"
+    if axis == 4:
+        return ("tile_pre" if flags & LG.PF_NOSTORE else "tile_gpe" if flags & LG.PF_MID_GPE else
+                "tile_pot" if flags & LG.PF_MID_POT else "tile_fft")
     if axis == 2 and flags & LG.PF_NOSTORE:
         return "z_inv_pre"
     if axis == 2 and nfft == 2 and flags & LG.PF_MID_GPE:
@@ -54,7 +59,8 @@ def pass_bytes_per_point(name, S):
     fused pointwise work reads or writes (vext 8 B, V_eff 8 B)."""
     return {"z_inv_pre": S + 8 + 8,  # S read (not stored), vext read, V_eff written
             "y_fft": 2 * S, "x_kin": 2 * S,
-            "z_gpe": 2 * S + 8}.get(name)  # V_eff read
+            "z_gpe": 2 * S + 8,  # V_eff read
+            "tile_pre": S + 8 + 8, "tile_kin": 2 * S, "tile_gpe": 2 * S + 8}.get(name)
 
 
 def insitu_passes(lib, LG, step_fn, steps, N, S):
@@ -156,15 +162,23 @@ PASS_SYMBOL = {name: f"256, {layout}, {kind}, HIP_vector_type<double, 2u>, false
                                           ("z_inv_pre", "true", 4))}
 
 
+# the same of the tile passes (libgrid_amd/csrc/hip/tile_pass.hpp): rows of 256 z and 16 l with real
+# factors; 256 x and 16 h, imaginary-time GPE and start of step
+TILE_SYMBOL = {"tile_kin": "tile_kinetic<HIP_vector_type<double, 2u>, 256, 16, true>",
+               "tile_gpe": "tile_potential<HIP_vector_type<double, 2u>, 256, 16, 3>",
+               "tile_pre": "tile_potential<HIP_vector_type<double, 2u>, 256, 16, 0>"}
+
+
 def profiled_traffic(pass_name, n):
     """HBM bytes per launch of a pass from the committed PMC summary (FETCH_SIZE + WRITE_SIZE,
     calibrated against the streaming copy), or None when it is not available for this pass."""
-    path = os.path.join(ROOT, "profiles", "gpe256_fft_pass_hbm_traffic.txt")
-    key = PASS_SYMBOL.get(pass_name)
+    tile = pass_name in TILE_SYMBOL
+    path = os.path.join(ROOT, "profiles", f"gpe256_{'tile' if tile else 'fft'}_pass_hbm_traffic.txt")
+    key = TILE_SYMBOL[pass_name] if tile else PASS_SYMBOL.get(pass_name)
     if n != 256 or key is None or not os.path.exists(path):
         return None
     for line in open(path):
-        if "fft_pass_kernel<HIP_vector_type<double, 2u>, " + key in line:
+        if (key if tile else "fft_pass_kernel<HIP_vector_type<double, 2u>, " + key) in line:
             parts = line.split()
             return (float(parts[0]) + float(parts[1])) * 1024 * 1024
     return None
@@ -562,12 +576,12 @@ def main():
         "data": "synthetic (seeded GPE barrier-trap state, random smoothed phase)",
         "config": {"workload": f"gpe_barrier {n}^3 complex128 imaginary-time split-operator step (dt 0.05, g 0.1, "
                                f"renormalised, start-of-step energy)", "grid": [n, n, n], "step_bohr": step,
-                   "passes_per_step": 8},
-        "roofline": {"bound": "hbm", "kernel": f"fft_pass {dname}", "achieved": d["gbps"], "peak": HBM_PEAK_GBPS,
+                   "passes_per_step": round(sum(v["count"] for v in kinds.values()))},
+        "roofline": {"bound": "hbm", "kernel": f"{'' if dname.startswith('tile') else 'fft_pass '}{dname}", "achieved": d["gbps"], "peak": HBM_PEAK_GBPS,
                      "unit": "GB/s", "frac": d["gbps"] / HBM_PEAK_GBPS, "traffic": traffic,
                      "algorithmic_bytes_per_launch": d["bytes"], "avg_launch_ms": d["ms"]},
-        # the step on the bytes it moves (264 B/pt: the deferred z transform cancels two z sweeps
-        # per step); the 400 B/pt model of a 12-sweep step is kept for reference only
+        # the step on the bytes it moves (136 B/pt: start, kinetic, potential, kinetic, the state kept
+        # transformed between steps); the 400 B/pt model of a 12-sweep step is kept for reference only
         "step_roofline": {"actual_bytes_per_step": actual_bytes,
                           "achieved_GBps": actual_bytes / (ms_step * 1e-3) / 1e9,
                           "frac": actual_bytes / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBPS,
