@@ -440,32 +440,53 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomA<C, LZ, B>::R>(), 8))) tile_kin
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = cscale(v[j], post);
   }
-  if constexpr (AY::TABLE) tile_sync<NT>();
-  AY::forward(v, tid, taby, lds);
-  exchange<typename AY::Last, typename AZ::First, C, R, NT, PD, PW>(v, tid, lds);
-  if constexpr (AZ::LDS) tile_sync<NT>();  // the waves' own exchanges reuse the buffer
-  AZ::forward(v, tid, tabz, lds);
-
   // kinetic factor: the last z digit is in registers.  The slots above this tile are M consecutive
   // (x, h) slots, or h slots in a 2-D grid; k1 is the frequency of the h slot, nh their number.
   using ZL = typename AZ::Last;
   constexpr int RZ = ZL::r, ZH = LZ / RZ;
   const int nh = a.nh, flat0 = (int)blockIdx.x * M;
   const double2 *t0 = (const double2 *)a.ktab_0, *t1 = (const double2 *)a.ktab_1, *t2 = (const double2 *)a.ktab_2;
-#pragma unroll
-  for (int u = 0; u < R / RZ; ++u) {
+  auto frequencies = [&](int u, int &k0, int &k1, int &kz) {
     const int lin = ZL::lin(tid, u), zs = (lin % LZ) / RZ, ys = (lin / LZ) % B;
-    const int kz = G::DZ.n == 3 ? zs / G::DZ.d[1] + G::DZ.d[0] * (zs % G::DZ.d[1]) : zs;
+    kz = G::DZ.n == 3 ? zs / G::DZ.d[1] + G::DZ.d[0] * (zs % G::DZ.d[1]) : zs;
     const int kl = slot_frequency(ys, G::DY.d[0], G::DY.d[1], G::DY.d[2]);
     const int flat = flat0 + (M == 1 ? 0 : lin / (LZ * B));
-    const int k0 = a.flat ? 0 : flat / nh, k1 = (a.flat ? flat : flat - k0 * nh) + nh * kl;
+    k0 = a.flat ? 0 : flat / nh;
+    k1 = (a.flat ? flat : flat - k0 * nh) + nh * kl;
+  };
+  auto outer = [&](int k0, int k1) { return REALK ? make_double2(t0[k0].x * t1[k1].x, 0.0) : cmul(t0[k0], t1[k1]); };
+  // tiles of 8 values, the small grids', load the tables with the tile: a launch there is a chain of
+  // latencies (with the same in the potential passes 32^3 FP64, 16 steps: 237 -> 231 us; steps of 16^3
+  // to 64^3 3 to 8 %)
+  constexpr bool EARLY = R <= 8;
+  double2 fxy[EARLY ? R / RZ : 1], fz[EARLY ? R : 1];
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int u = 0; u < R / RZ; ++u) {
+      int k0, k1, kz;
+      frequencies(u, k0, k1, kz);
+      fxy[u] = outer(k0, k1);
+#pragma unroll
+      for (int i = 0; i < RZ; ++i) fz[u * RZ + i] = REALK ? make_double2(t2[kz + ZH * i].x, 0.0) : t2[kz + ZH * i];
+    }
+  }
+  if constexpr (AY::TABLE) tile_sync<NT>();
+  AY::forward(v, tid, taby, lds);
+  exchange<typename AY::Last, typename AZ::First, C, R, NT, PD, PW>(v, tid, lds);
+  if constexpr (AZ::LDS) tile_sync<NT>();  // the waves' own exchanges reuse the buffer
+  AZ::forward(v, tid, tabz, lds);
+
+#pragma unroll
+  for (int u = 0; u < R / RZ; ++u) {
+    int k0, k1, kz;
+    frequencies(u, k0, k1, kz);
     if (fl & HGRID_PF_MID_KRED) {
       const double kk = a.k2_0[k0] + a.k2_1[k1];
 #pragma unroll
       for (int i = 0; i < RZ; ++i) acc[HGRID_RED_KIN] += (kk + k2_of<LZ>(kz + ZH * i, a.k2_dk)) * cnorm2(v[u * RZ + i]);
     }
     // factors in groups of four behind scheduling fences, so that few are live at once
-    const double2 f = REALK ? make_double2(t0[k0].x * t1[k1].x, 0.0) : cmul(t0[k0], t1[k1]);
+    const double2 f = EARLY ? fxy[EARLY ? u : 0] : outer(k0, k1);
 #pragma unroll
     for (int i0 = 0; i0 < RZ; i0 += 4) {
       __builtin_amdgcn_sched_barrier(0);
@@ -475,9 +496,9 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomA<C, LZ, B>::R>(), 8))) tile_kin
           // hidden from the sum above, with which the compiler would share the values widened to FP64,
           // all at once (FP32, rows of 512: 145 registers spilled)
           if constexpr (sizeof(C) == 8) asm volatile("" : "+v"(v[u * RZ + i].x), "+v"(v[u * RZ + i].y));
-          v[u * RZ + i] = cscale_d(v[u * RZ + i], t2[kz + ZH * i].x * f.x);
+          v[u * RZ + i] = cscale_d(v[u * RZ + i], (EARLY ? fz[EARLY ? u * RZ + i : 0].x : t2[kz + ZH * i].x) * f.x);
         }
-        else v[u * RZ + i] = cmul(v[u * RZ + i], round_to<C>(cmul(t2[kz + ZH * i], f)));
+        else v[u * RZ + i] = cmul(v[u * RZ + i], round_to<C>(cmul(EARLY ? fz[EARLY ? u * RZ + i : 0] : t2[kz + ZH * i], f)));
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -640,11 +661,13 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   auto potential_offset = [&](int t, int u) { return ordered ? (unsigned)(u * SV::r * NT + t) * 8u : real_element(t, u) * 8u; };
   // the start-of-step pass loads vext ahead of the exchange, which hides the latency (256^3 FP64
   // 160 -> 147 us); the potential passes have no registers for it
-  // 1024 threads of 32 values have no registers for the potential of all of them
-  constexpr bool FULL = NT == 1024 && R == 32;
-  double pv[KIND == TPRE && !FULL ? R : 1];
+  // 1024 threads of 32 values have no registers for the potential of all of them; tiles of 8 values,
+  // the small grids', load it with the tile in every kind
+  constexpr bool FULL = NT == 1024 && R == 32, EARLY = R <= 8;
+  constexpr bool EARLYV = EARLY && (KIND == TGPE || KIND == TGPR);
+  double pv[(KIND == TPRE && !FULL) || EARLYV ? R : 1];
   auto load_potential = [&]() {
-    if constexpr (KIND == TPRE && !FULL) {
+    if constexpr ((KIND == TPRE && !FULL) || EARLYV) {
 #pragma unroll
       for (int u = 0; u < R / SV::r; ++u) {
         const unsigned e = potential_offset(tid, u);
@@ -653,11 +676,23 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
       }
     }
   };
+  // another array's value at the thread's real-space element j
+  auto value_of = [&](__amdgpu_buffer_rsrc_t array, int j) {
+    return bload<C>(array, real_element(tid, j / SV::r) * CS, (unsigned)(j % SV::r) * stepv * CS);
+  };
+  C early[EARLY && (KIND == TPOT || KIND == TMRG) ? R : 1];
+  if constexpr (EARLY && (KIND == TPOT || KIND == TMRG)) {
+    const void *array = KIND == TPOT ? a.pot : a.merge;
+    const auto ro = make_rsrc(array, array ? ntot * CS : 0);
+#pragma unroll
+    for (int j = 0; j < R; ++j) early[j] = value_of(ro, j);
+  }
+  if constexpr (EARLYV) load_potential();
   if (!skip1) {
     conj_all(v);
     if constexpr (A == 1) split_twiddle();
     AX::inverse(v, tid, tabx, lds);
-    load_potential();
+    if constexpr (KIND == TPRE) load_potential();
     if constexpr (A > 1) {
       exchange<X0, SV, C, R, NT, PD, PW>(v, tid, lds);
       split_twiddle();
@@ -670,7 +705,7 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
 #pragma unroll
       for (int j = 0; j < R; ++j) asm volatile("" : "+v"(v[j].x), "+v"(v[j].y));
     }
-  } else {
+  } else if constexpr (KIND == TPRE) {
     load_potential();
   }
 
@@ -697,15 +732,17 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
   } else if constexpr (KIND == TPOT || KIND == TMRG) {
     // values of another array at the tile's real-space elements, four ahead of their use
     auto with_values = [&](const void *array, auto &&apply) {
+      if constexpr (EARLY) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = apply(v[j], early[j], j / SV::r, j % SV::r);
+        return;
+      }
       const auto ro = make_rsrc(array, ntot * CS);
       constexpr int AHEAD = R % 4 == 0 ? 4 : R;
       C p[2][AHEAD];
       auto fetch = [&](int j0, C(&q)[AHEAD]) {
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j) {
-          const int u = (j0 + j) / SV::r, i = (j0 + j) % SV::r;
-          q[j] = bload<C>(ro, real_element(tid, u) * CS, (unsigned)i * stepv * CS);
-        }
+        for (int j = 0; j < AHEAD; ++j) q[j] = value_of(ro, j0 + j);
       };
       fetch(0, p[0]);
 #pragma unroll
@@ -753,7 +790,7 @@ __attribute__((amdgpu_waves_per_eu(waves<C, GeomB<C, LX, A>::R>(), 8))) tile_pot
         double p[SV::r];
         auto fetch = [&](int i0, int n) {
 #pragma unroll
-          for (int i = i0; i < i0 + n; ++i) p[i] = a.cons + bload_f64(rpv, e, (unsigned)i * steppv);
+          for (int i = i0; i < i0 + n; ++i) p[i] = a.cons + (EARLY ? pv[EARLY ? u * SV::r + i : 0] : bload_f64(rpv, e, (unsigned)i * steppv));
         };
         if constexpr (!FULL) fetch(0, SV::r);
 #pragma unroll
