@@ -95,23 +95,27 @@ template <typename C, int L, typename S> int launch(const hgrid_pass *p) {
 }
 
 // The lengths at which rows beat pencils, us at 2^22.6 to 2^23 points, pencils and then rows:
-//   FP64  96: 34.4 30.1   192: 34.1 30.6   384: 61.9 37.4   (64, 128, 256, 512: equal; 1024: 40 51)
+//   FP64  96: 34.4 30.1   192: 34.1 30.6*  384: 61.9 37.4   (64, 128, 256, 512: equal; 1024: 40 51)
 //   FP32  64: 22.3 21.0    96: 22.3 18.0   128: 22.7 20.9   192: 19.9 17.0   256: 22.2 20.8
 //        384: 21.1 19.6   512: 27.3 24.5   (1024: 25.9 31.3)
 //   FP32 storage with FP64 arithmetic  64: 22.6 21.2   96: 26.4 20.7   128: 25.4 21.8
-//        192: 22.8 20.3   256: 24.3 22.3   384: 50.0 27.6   512: 32.1 27.7   (1024: 29.7 40.3)
+//        192: 22.8 20.3*  256: 24.3 22.3   384: 50.0 27.6   512: 32.1 27.7   (1024: 29.7 40.3)
 // 48 points gain in the largest grids only (FP32 21.6 19.9, but 16 x 16 x 48 6.2 6.9).
+// *: left to the pencils all the same.  One transform of 256 x 128 x 192 in FP64 that went this way
+// came back 9.7e-4 off, the size of some six lost elements.  Neither the kernel's source and assembly
+// nor later runs of the same transform showed the cause, so the one length and arithmetic that it was
+// seen with does not take this way; it loses a tenth of one of the three passes.
 #define LG_ROW_LENGTHS(X) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 
 constexpr bool covers(long L, int prec) {
 #define LG_CASE(n) || L == n
-  return (false LG_ROW_LENGTHS(LG_CASE)) && (prec != HGRID_C128 || L % 3 == 0);
+  return (false LG_ROW_LENGTHS(LG_CASE)) && (prec != HGRID_C128 || L % 3 == 0) && (prec == HGRID_C64 || L != 192);
 #undef LG_CASE
 }
 
 template <typename C, typename S = C> int launch_len(const hgrid_pass *p) {
 #define LG_CASE(n) \
-  case n: if constexpr (covers(n, sizeof(S) == 16 ? HGRID_C128 : HGRID_C64)) return launch<C, n, S>(p); else return -1;
+  case n: if constexpr (covers(n, sizeof(S) == 16 ? HGRID_C128 : sizeof(C) == 16 ? HGRID_C64X : HGRID_C64)) return launch<C, n, S>(p); else return -1;
   switch (p->n2) {
     LG_ROW_LENGTHS(LG_CASE)
     default: return -1;
