@@ -853,8 +853,10 @@ void grid_wf_propagate(wf *gwf, cgrid *potential, REAL complex time) {
     if (!gwf->cworkspace)
       gwf->cworkspace = cgrid_alloc(g->nx, g->ny, g->nz, g->step, g->value_outside, g->outside_params_ptr, "WF cworkspace 1");
     cgrid *w = gwf->cworkspace;
+    /* the copy's own refusal, ahead of the form of the step that makes none */
+    if (w->nx != g->nx || w->ny != g->ny || w->nz != g->nz) lg_fatal("Incompatible grids in cgrid_copy().");
     if (cgrid_get_precision(w) != cgrid_get_precision(g)) cgrid_set_precision(w, cgrid_get_precision(g));
-    if (lg_cdev(g) && w != potential && g != potential) {
+    if (lg_cdev(g) && w != g && w != potential && g != potential) {
       check_fft_grid(g);
       step_args args[2];
       split_args(gwf, potential, time, &args[0]);
