@@ -837,7 +837,9 @@ static int tile_absorb_step(wf *gwf, cgrid *w, const step_args *args) {
   lg_run_tile(&t, HGRID_TILE_MERGE);
   lg_c_written(g, 1);
   d->zpend = 2;
+  /* the workspace holds the imaginary-time state, in tile form too: who reads it sees that state */
   lg_c_written(w, 1);
+  w->dev->zpend = 2;
   return 1;
 }
 

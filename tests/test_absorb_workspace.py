@@ -66,3 +66,18 @@ def test_grid_as_its_own_workspace(lg, shape):
     got, _ = stepped(lg, psi, pot, b"\x00", (0.02,), bounds, own=True)
     want, _ = stepped(lg, psi, pot, b"\x00", (0.02, -0.02j))
     assert rel_l2(got, want) < 2e-14
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,bar", [(b"\x00", 2e-14), (b"\x01", 1e-5)])
+@pytest.mark.parametrize("shape", [(16, 32, 24), (48, 64, 16), (16, 8, 16), (1, 32, 16)])
+def test_workspace_holds_the_imaginary_time_state(lg, shape, prec, bar):
+    """After one step, and after two, the workspace reads as the imaginary-time step of the state that the
+    last step began with, in tile passes and in pencils.  Bars of test_tile_pass.py."""
+    psi, pot, bounds = inputs(shape)
+    first, work = stepped(lg, psi, pot, prec, (0.02,), bounds)
+    want, _ = stepped(lg, psi, pot, prec, (-0.02j,))
+    assert rel_l2(work, want) < bar
+    _, work = stepped(lg, psi, pot, prec, (0.02, 0.02), bounds)
+    want, _ = stepped(lg, first, pot, prec, (-0.02j,))
+    assert rel_l2(work, want) < bar
