@@ -212,20 +212,30 @@ void *lg_c_raw(cgrid *g, const double **scale) {
   return d->d;
 }
 
-void *lg_c_in(cgrid *g, const double **scale) {
-  grid_dev *d = lg_cdev(g);
-  if (!(d->valid & GV_DEV)) upload(g);
-  if (!scale && d->pending && d->zpend) {
+/* real space with no pending scale */
+static void settle(cgrid *g) {
+  grid_dev *d = g->dev;
+  if (d->pending && d->zpend) {
     /* the inverse transform applies the pending scale */
     inverse_into(g, d->d, d->dscal + GS_SCALE);
     d->zpend = 0;
     scale_applied(d);
     d->valid = GV_DEV;
+    return;
+  }
+  lg_c_materialize(g);
+  lg_c_flush(g);
+}
+
+void *lg_c_in(cgrid *g, const double **scale) {
+  grid_dev *d = lg_cdev(g);
+  if (!(d->valid & GV_DEV)) upload(g);
+  if (!scale) {
+    settle(g);
     return d->d;
   }
   lg_c_materialize(g);
-  if (scale) *scale = d->pending ? d->dscal + GS_SCALE : NULL;
-  else if (d->pending) lg_c_flush(g);
+  *scale = d->pending ? d->dscal + GS_SCALE : NULL;
   return d->d;
 }
 
@@ -295,7 +305,7 @@ void lg_c_flush(cgrid *g) {
 void lg_c_host_sync(cgrid *g) {
   grid_dev *d = g->dev;
   if (d->valid & GV_HOST) return;
-  lg_c_in_flushed(g);
+  settle(g); /* also of a grid that has been locked to the host since: its values can still be read */
   download(g);
 }
 
