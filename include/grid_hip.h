@@ -339,6 +339,7 @@ int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void *w, const 
  * rows. */
 int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, const void *x, int xs, int xo, int cin, int lgS,
                          long nvox, float *partial, float *bpartial);
+long hgrid_nn_wgrad_chunk(long nvox, int lgS); /* voxels per chunk */
 long hgrid_nn_wgrad_chunks(long nvox, int lgS);
 long hgrid_nn_wgrad_partials(long nvox, int lgS);
 int hgrid_nn_reduce(const float *partial, long np, long n, float *out, int accumulate);

@@ -143,16 +143,99 @@ __global__ void __launch_bounds__(256) k_conv3(const bf16 *__restrict__ x, int x
     }
 }
 
+// The same for any number of channels and any cube: what the table's entries and the packed coordinates
+// of k_conv3 do not hold (more than 192 channels, sides beyond 1024).  Each chunk's tap and channels are
+// counted along and its neighbour formed coordinate by coordinate.
+template <int MT, int NTL>
+__global__ void __launch_bounds__(256) k_conv3_any(const bf16 *__restrict__ x, int xs, int xo, int cin,
+                                                   const bf16 *__restrict__ w, const float *__restrict__ bias,
+                                                   bf16 *__restrict__ y, int ys, int yo, const bf16 *__restrict__ mask,
+                                                   int mks, int mko, int lgS, long nvox, int relu) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, r = lane & 15;
+  const long m0 = ((long)blockIdx.x * 4 + wave) * (16 * MT);
+  const int co0 = blockIdx.y * (16 * NTL);
+  const int msk = (1 << lgS) - 1;
+  const int nch = 27 * (cin >> 3);
+  long vb[MT];
+  int vz[MT], vy[MT], vx[MT];
+  bool vok[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const long m = m0 + 16 * mt + r;
+    vok[mt] = m < nvox;
+    const long mm = vok[mt] ? m : 0;
+    vx[mt] = (int)(mm & msk);
+    vy[mt] = (int)((mm >> lgS) & msk);
+    vz[mt] = (int)((mm >> (2 * lgS)) & msk);
+    vb[mt] = (mm >> (3 * lgS)) << (3 * lgS);
+  }
+  f32x4 acc[MT][NTL];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NTL; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // chunk kc + g of every step: (tap, channel block cb)
+  int tap = 0, cb = 8 * g;
+  while (cb >= cin) {
+    cb -= cin;
+    ++tap;
+  }
+  const long wrow = 27L * cin;
+#pragma unroll 1
+  for (int kc = 0; kc < nch; kc += 4) {
+    const bool cok = tap < 27;
+    bf16x8 a[MT], bw[NTL];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      a[mt] = zero8();
+      if (cok && vok[mt]) a[mt] = ld8(x + nbr(vb[mt], vz[mt], vy[mt], vx[mt], tap, lgS) * xs + xo + cb);
+    }
+#pragma unroll
+    for (int j = 0; j < NTL; ++j) {
+      bw[j] = zero8();
+      if (cok) bw[j] = ld8(w + (long)(co0 + 16 * j + r) * wrow + (long)tap * cin + cb);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int j = 0; j < NTL; ++j) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bw[j], acc[mt][j], 0, 0, 0);
+    cb += 32;
+    while (cb >= cin) {
+      cb -= cin;
+      ++tap;
+    }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NTL; ++j) {
+      const int co = co0 + 16 * j + r;
+      const float bv = bias ? bias[co] : 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long m = m0 + 16 * mt + 4 * g + i;
+        if (m < nvox) {
+          float v = acc[mt][j][i] + bv;
+          if (relu) v = fmaxf(v, 0.f);
+          if (mask && !(f(mask[m * mks + mko + co]) > 0.f)) v = 0.f;
+          y[m * ys + yo + co] = b(v);
+        }
+      }
+    }
+}
+
 // ---- weight gradient: dW[co][t][ci] = sum_m dY[m][co] X[m + d_t][ci] ----------------------
 // Grid (chunks, 27 taps, Cout / (16 CT)).  A workgroup stages 128 voxels of dY (16 CT channels)
 // and of X at the tap's neighbours into LDS transposed to [channel][voxel], then each wave
 // takes 32 of the voxels as the K of one MFMA per (co tile, ci tile).  Every wave writes its
-// own partial sums (no atomics); k_reduce adds the partials in a fixed order.
+// own partial sums (no atomics), or with ONE the waves' sums are added through LDS in their order and
+// a chunk writes one partial, as k_wgrad_rows does; k_reduce adds the partials in a fixed order.
 constexpr int WG_V = 128;       // voxels staged per step
 constexpr int WG_P = WG_V + 8;  // LDS row pitch (bf16): 16 rows of a b128 read hit 16 distinct bank groups
 constexpr int WG_MAXT = 12;     // ci tiles (Cin <= 192)
 
-template <int CT>
+template <int CT, bool ONE>
 __global__ void __launch_bounds__(256) k_conv3_wgrad(const bf16 *__restrict__ dy, int dys, int dyo,
                                                      const bf16 *__restrict__ x, int xs, int xo, int cin, int lgS,
                                                      long nvox, long vc, int cout, float *__restrict__ partial,
@@ -222,8 +305,28 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad(const bf16 *__restrict__ dy
     }
   }
   if (bias_wg && threadIdx.x < 16 * CT) bpartial[(long)blockIdx.x * cout + co0 + threadIdx.x] = bsum;
-  // partial[(chunk * 4 + wave)][co][tap][ci]
-  float *pp = partial + ((long)blockIdx.x * 4 + wave) * ((long)cout * 27 * cin);
+  if constexpr (ONE) {
+    float *sum = (float *)xs_;  // [co tile][ci tile][lane][4]
+    static_assert(CT * WG_MAXT * 256 * sizeof(float) <= sizeof(xs_), "room for the waves' sums");
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+      __syncthreads();
+      if (wave == k) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int j = 0; j < WG_MAXT; ++j)
+            if (j < ntile) {
+              f32x4 *t = (f32x4 *)(sum + ((c * WG_MAXT + j) * 64 + lane) * 4);
+              acc[c][j] += k ? *t : f32x4{0.f, 0.f, 0.f, 0.f};
+              *t = acc[c][j];
+            }
+      }
+    }
+    if (wave != 3) return;  // the last wave holds the sums of all
+  }
+  // partial[(chunk * 4 + wave)][co][tap][ci]; ONE: [chunk][co][tap][ci]
+  float *pp = partial + (ONE ? (long)blockIdx.x : (long)blockIdx.x * 4 + wave) * ((long)cout * 27 * cin);
 #pragma unroll
   for (int c = 0; c < CT; ++c)
 #pragma unroll
@@ -749,7 +852,6 @@ extern "C" int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void
       nvox <= 0 || nvox % (1L << (3 * lgS)))
     return lg::fail("nn_conv3: shape");
   if (((uintptr_t)x | (uintptr_t)w) & 15) return lg::fail("nn_conv3: operands must be 16-byte aligned");
-  if (cin > 192 || lgS > 10) return lg::fail("nn_conv3: shape");
   // tiles of 2 or 4 voxel groups x up to 4 channel groups share operands; where that leaves fewer than
   // 1024 waves (four per CU) single tiles make more of them, and the operands are fetched two steps
   // ahead, which larger grids cannot afford in registers (48 -> 16 channels, 8 x 64^3: 460 us without,
@@ -757,24 +859,31 @@ extern "C" int hgrid_nn_conv3(const void *x, int xs, int xo, int cin, const void
   const int t16 = cout / 16;
   int ntl = t16 % 4 == 0 ? 4 : t16 % 3 == 0 ? 3 : t16 % 2 == 0 ? 2 : 1;
   int mt = ntl == 1 ? 4 : 2;
-  if (nvox / (16 * mt) * (t16 / ntl) < 1024) ntl = mt = 1;
+  const bool any = cin > 192 || lgS > 10;  // beyond the table and the packed coordinates
+  if (!any && nvox / (16 * mt) * (t16 / ntl) < 1024) ntl = mt = 1;
   dim3 grid(blocks(nvox, 64 * mt), t16 / ntl);
   auto *X = (const bf16 *)x;
   auto *W = (const bf16 *)w;
   auto *Y = (bf16 *)y;
   auto *M = (const bf16 *)mask;
-#define LG_CONV(mtv, ntlv, depth) \
-  hipLaunchKernelGGL((k_conv3<mtv, ntlv, depth>), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu)
-  if (ntl == 4) LG_CONV(2, 4, 1);
-  else if (ntl == 3) LG_CONV(2, 3, 1);
-  else if (ntl == 2) LG_CONV(2, 2, 1);
-  else if (mt == 4) LG_CONV(4, 1, 1);
-  else LG_CONV(1, 1, 3);
+#define LG_CONV(...) \
+  hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(256), 0, lg::stream(), X, xs, xo, cin, W, bias, Y, ys, yo, M, mks, mko, lgS, nvox, relu)
+  if (any) {
+    if (ntl == 4) LG_CONV(k_conv3_any<2, 4>);
+    else if (ntl == 3) LG_CONV(k_conv3_any<2, 3>);
+    else if (ntl == 2) LG_CONV(k_conv3_any<2, 2>);
+    else LG_CONV(k_conv3_any<4, 1>);
+  } else if (ntl == 4) LG_CONV(k_conv3<2, 4, 1>);
+  else if (ntl == 3) LG_CONV(k_conv3<2, 3, 1>);
+  else if (ntl == 2) LG_CONV(k_conv3<2, 2, 1>);
+  else if (mt == 4) LG_CONV(k_conv3<4, 1, 1>);
+  else LG_CONV(k_conv3<1, 1, 3>);
 #undef LG_CONV
   return lg::check_launch("nn_conv3");
 }
 
-// the cubes of k_wgrad_rows; other sides keep the tap-by-tap kernel
+// the cubes of k_wgrad_rows; other sides keep the tap-by-tap kernel, and so do, on these cubes, channels
+// in other counts than 8 and multiples of 16, operands off 16 bytes and part of a cube
 static bool wgrad_by_rows(int lgS) { return lgS >= 3 && lgS <= 6; }
 
 // voxels per workgroup: a multiple of 256.  By rows, 1024 or so (256 in the smallest layers, and at
@@ -789,6 +898,8 @@ static long wgrad_chunk(long nvox, int lgS) {
   const long vc = ((nvox + n - 1) / n + 255) / 256 * 256;
   return vc;
 }
+
+extern "C" long hgrid_nn_wgrad_chunk(long nvox, int lgS) { return wgrad_chunk(nvox, lgS); }
 
 extern "C" long hgrid_nn_wgrad_chunks(long nvox, int lgS) {
   const long vc = wgrad_chunk(nvox, lgS);
@@ -818,9 +929,9 @@ extern "C" int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, 
   const unsigned chunks = (unsigned)((nvox + vc - 1) / vc);
   auto *D = (const bf16 *)dy;
   auto *X = (const bf16 *)x;
-  if (wgrad_by_rows(lgS)) {
-    if (nvox % (1L << (3 * lgS)) || (cin % 16 && cin != 8) || ((uintptr_t)dy | (uintptr_t)x) & 15 || (dys | dyo | xs | xo) & 7)
-      return lg::fail("nn_conv3_wgrad: shape");
+  const bool one = wgrad_by_rows(lgS);  // one partial a chunk
+  if (one && nvox % (1L << (3 * lgS)) == 0 && (cin == 8 || (cin > 0 && cin % 16 == 0)) &&
+      !(((uintptr_t)dy | (uintptr_t)x) & 15) && !((dys | dyo | xs | xo) & 7)) {
     dim3 grid(chunks, (cin + 15) / 16, t16 / ct);
     switch (lgS) {
       case 3: launch_wgrad_rows<3>(grid, ct, D, dys, dyo, X, xs, xo, cin, nvox, vc, cout, partial, bpartial); break;
@@ -831,10 +942,16 @@ extern "C" int hgrid_nn_conv3_wgrad(const void *dy, int dys, int dyo, int cout, 
     return lg::check_launch("nn_conv3_wgrad");
   }
   dim3 grid(chunks, 27, t16 / ct);
-  switch (ct) {
-    case 2: hipLaunchKernelGGL((k_conv3_wgrad<2>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, lgS, nvox, vc, cout, partial, bpartial); break;
-    default: hipLaunchKernelGGL((k_conv3_wgrad<1>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, lgS, nvox, vc, cout, partial, bpartial); break;
+#define LG_WGRAD(ctv, onev) \
+  hipLaunchKernelGGL((k_conv3_wgrad<ctv, onev>), grid, dim3(256), 0, lg::stream(), D, dys, dyo, X, xs, xo, cin, lgS, nvox, vc, cout, partial, bpartial)
+  if (ct == 2) {
+    if (one) LG_WGRAD(2, true);
+    else LG_WGRAD(2, false);
+  } else {
+    if (one) LG_WGRAD(1, true);
+    else LG_WGRAD(1, false);
   }
+#undef LG_WGRAD
   return lg::check_launch("nn_conv3_wgrad");
 }
 
