@@ -8,6 +8,7 @@
  * the convergence measure) repeated until the energy is converged to tol by the rule of the
  * host relaxation (relax_rule.h), with that relaxation's vector extrapolation.
  */
+#include <stdint.h>
 #include <sys/stat.h>
 #include <unistd.h>
 
@@ -117,6 +118,18 @@ static void b2d_free(b2d_batch *b) {
 static int cmp_desc(const void *a, const void *b) {
   const long *x = (const long *)a, *y = (const long *)b;
   return (x[0] < y[0]) - (x[0] > y[0]);
+}
+
+/* a problem's grid and its place in the call: by grid, then by place */
+typedef struct {
+  cgrid *grid;
+  INT i;
+} b2d_target;
+
+static int cmp_target(const void *a, const void *b) {
+  const b2d_target *x = (const b2d_target *)a, *y = (const b2d_target *)b;
+  if (x->grid != y->grid) return (uintptr_t)x->grid < (uintptr_t)y->grid ? -1 : 1;
+  return (x->i > y->i) - (x->i < y->i);
 }
 
 static void b2d_pack(b2d_batch *b, INT ns, wf **gwf, rgrid **pot, REAL dt, REAL tol, INT max_steps, INT stride) {
@@ -376,12 +389,19 @@ REAL grid_wf_batch2d_relax(INT nsolves, wf **gwf, rgrid **potential, REAL dt, RE
   }
   float *hpsi = (float *)malloc(sizeof(float) * 2 * b.total);
   lg_hip(hgrid_memcpy_d2h(hpsi, b.psi_pool, sizeof(float) * 2 * b.total), "hipMemcpy (batch psi)");
+  /* the states are unpacked side by side; a grid that was given several times takes its last problem's */
+  b2d_target *to = (b2d_target *)malloc(sizeof(b2d_target) * (size_t)nsolves);
+  if (!to) lg_fatal("out of host memory (batched solves)");
+  for (INT i = 0; i < nsolves; ++i) to[i] = (b2d_target){gwf[i]->grid, i};
+  qsort(to, nsolves, sizeof(b2d_target), cmp_target);
 #pragma omp parallel for schedule(dynamic, 1)
-  for (INT i = 0; i < nsolves; ++i) {
-    cgrid *g = gwf[i]->grid;
-    const long nn = g->ny * g->nz, o = b.off[i];
+  for (INT r = 0; r < nsolves; ++r) {
+    cgrid *g = to[r].grid;
+    if (r + 1 < nsolves && to[r + 1].grid == g) continue;
+    const long nn = g->ny * g->nz, o = b.off[to[r].i];
     for (long k = 0; k < nn; ++k) g->value[k] = (double)hpsi[2 * (o + k)] + I * (double)hpsi[2 * (o + k) + 1];
   }
+  free(to);
   for (INT i = 0; i < nsolves; ++i) {
     cgrid *g = gwf[i]->grid;
     cgrid_host_modified(g);
