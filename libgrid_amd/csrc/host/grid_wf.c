@@ -390,7 +390,7 @@ static int tile_step(wf *gwf, const step_args *sa) {
     hgrid_reduce_job j = {partB, nbB, HGRID_RED_NORM, 3, d->dscal + GS_RED};
     fin.job[fin.njobs++] = j;
   }
-  const int hand_on = (stage == 1 || stage == 2) && sa->want_post_norm && sa->renorm_target > 0.0 && nbB <= 4096;
+  const int hand_on = (stage == 1 || stage == 2) && sa->want_post_norm && sa->renorm_target > 0.0;
   long nbpost = nbA;
   for (int half = 0; half < 2; ++half) {
     if ((stage == 1 || stage == 2) && half == 1) break;
