@@ -153,8 +153,9 @@ def fp64_512_bench(lib, LG, steps=10, warmup=3):
     return out
 
 
-# template instantiation of each pass of the 256^3 FP64 imaginary-time step in the rocprofv3
-# summaries (length, contiguous, kernel kind, storage type, wide tiles): the kinds of
+# template instantiation of each pass of the 256^3 FP64 imaginary-time step in pencil passes, which the
+# library took there before the tile passes below: what the committed summaries of that form name.  In
+# the rocprofv3 summaries (length, contiguous, kernel kind, storage type, wide tiles): the kinds of
 # libgrid_amd/csrc/hip/fft_pass.hpp are 8 plain transform (y), 6 real kinetic factors (x),
 # 5 imaginary-time GPE (z), 4 start-of-step (z)
 PASS_SYMBOL = {name: f"256, {layout}, {kind}, HIP_vector_type<double, 2u>, false>"
