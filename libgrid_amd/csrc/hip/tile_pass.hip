@@ -101,6 +101,11 @@ template <typename C> static bool plan(hgrid_tile *t) {
   //   FP64  256 192 512 (   512,    512)          7.7  7.4   6.9  6.2    9.2 10.6   22.2 23.2
   //         512 384 128 (   512,    512)          9.8  7.7   9.0  6.3   11.5 11.1   27.8 24.7
   //         192 512 256 (  1024,    256)          7.8  6.4   7.2  5.6    9.6 10.4   22.1 21.7
+  // `pencils` tells steps that end in real space and merged relaxations apart, not GPE steps from those with
+  // a complex potential.  The first line therefore leaves whole FP32 shapes to the pencils where the GPE step gains
+  // nothing or little (its 512 384 192 gains 7 %), although complex potentials would gain there.  384 points
+  // along z run better in tiles than the other long axes do, and an h with a factor 3 worse: these
+  // exceptions rest on the rows above alone.
   const bool f64 = sizeof(C) == 16;
   const int threads = t->threads_a + t->threads_b;
   if (!f64 && t->n2 != 384 && t->n1 >= 384 && t->threads_a >= 512 && t->threads_b >= 512) return false;

@@ -440,7 +440,9 @@ void cgrid_copy(cgrid *dst, cgrid *src) {
   if (sd->zpend && (sd->valid & GV_DEV) && dd->prec == sd->prec) {
     /* a state between fused steps: its inverse transform goes straight into the copy, with the pending
      * scale, and the state stays as the next step takes it (a snapshot then costs one sweep, not
-     * the transform, the scale, the copy and the way back into the step's form) */
+     * the transform, the scale, the copy and the way back into the step's form).  Each further copy of the
+     * same state costs that sweep again, where a state brought back would be copied plainly: 256^3 FP64
+     * 190 against 100 us, so four copies between two steps are where the two ways meet */
     lg_cdev(src);
     void *o = lg_c_out(dst);
     inverse_into(src, o, sd->pending ? sd->dscal + GS_SCALE : NULL);
